@@ -109,6 +109,7 @@ extern "C" int cupss_system_destroy(cupss_system s)
     if (s->stream) hipStreamSynchronize(s->stream);
     s->pending = nullptr;  // only the system's own batch can still hold it
     fused_release(s);
+    line_release(s);
     if (s->gexec) hipGraphExecDestroy(s->gexec);
     if (s->graph) hipGraphDestroy(s->graph);
     for (auto &F : s->f) {
@@ -770,6 +771,8 @@ extern "C" int cupss_system_advance(cupss_system s, int nsteps)
         }
         return fused_steps(s, nsteps);
     }
+    // 1D: the step program in one workgroup, whatever its fields and terms
+    if (s->path_mode == 0 && !hooks_present(s) && line_eligible(s)) return line_steps(s, nsteps);
     return general_advance(s, nsteps);
 }
 
@@ -812,6 +815,7 @@ extern "C" int cupss_system_device_bytes(cupss_system s, size_t *bytes)
         b += spec * (2 * s->plan.real.size() + s->plan.groups.size());
     else if (s->plan.ok)  // the fused path's buffers, allocated at its first run
         b += spec * (2 + 2 * s->plan.cons.size() + s->plan.real.size() + s->plan.groups.size());
+    b += line_device_bytes(s);
     *bytes = b;
     return CUPSS_OK;
 }

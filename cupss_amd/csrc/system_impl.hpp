@@ -113,6 +113,7 @@ struct cupss_system_t {
     uint64_t step = 0;
     int device = 0;
     void *batch = nullptr;    // internal one-instance fused batch
+    void *line = nullptr;     // one-workgroup program of a 1D system (line.hip)
     // The fused batch (internal or a cupss_batch's) whose last run left this
     // system's state column-major only: its transpose back to the natural
     // layout is deferred until something reads or writes the state outside
@@ -153,6 +154,12 @@ void fused_release(cupss_system s);
 // write back the natural-layout state that a fused run deferred (see
 // cupss_system_t::pending); no-op when nothing is pending
 int fused_flush(cupss_system s);
+// 1D systems (line.hip): whether the one-workgroup kernel takes the system's
+// program, and nsteps steps of it (the same semantics as general_steps)
+bool line_eligible(cupss_system s);
+int line_steps(cupss_system s, int nsteps);
+void line_release(cupss_system s);
+size_t line_device_bytes(cupss_system s);  // descriptor and tables, made at the first such run
 int fused_profile(cupss_system s, int on);
 int fused_kernel_time(cupss_system s, float *avg_ms, double *points, char *name, int len);
 }  // namespace cupss
