@@ -91,6 +91,7 @@ struct FusedBatch {
         int nc = 0, ny = 0;
         bool real = false;      // any instance has real fields (prologue)
         int width = 3;          // real fields the row kernel holds at once (fused_row_width)
+        bool lean = false;      // simple instances: the lean kernels
         int cons = 0;           // stored fields of the instances: 1 = constraints, 2 = dynamic fields too
         std::vector<int> insts;
         int lpb = 0, twd = 0;   // tile shapes
@@ -278,6 +279,82 @@ static bool step0_zero(cupss_system s, int f)
     return false;
 }
 
+// one prefactor of the pool as a lean operator; false where it is not a
+// monomial without 1/|q| (qz does not occur in 2D)
+static bool lean_op(const FusedInst &a, const TermRefDev &R, LeanOp &O)
+{
+    if (R.npres != 1) return false;
+    const PresDev &D = a.pool[R.pres0];
+    if (D.invq != 0 || D.cz != 0 || D.q2n < 0 || D.a < 0 || D.b < 0) return false;
+    O.c = D.c;
+    O.q2n = D.q2n;
+    O.a = D.a;
+    O.b = D.b;
+    O.mult_i = R.mult_i;
+    return true;
+}
+
+// the lean program of a finished 2D descriptor (FusedLean); false where the
+// system is not one
+static bool make_lean(FusedInst &a)
+{
+    FusedLean &P = a.lean;
+    if (a.ncons != 0 || a.ngroups > 1 || a.nreal > 2 || a.u.noise_invq != 0 || a.u.noise_q2n < 0) return false;
+    P.sy = a.g.sy;
+    P.nc = a.g.nc;
+    P.nc1 = a.g.nc1;
+    P.sqx = a.g.sqx;
+    P.sqy = a.g.sqy;
+    P.scale = a.scale;
+    P.dt = a.u.dt;
+    P.nreal = a.nreal;
+    P.ngroups = a.ngroups;
+    P.X = a.X[0];
+    P.eta = a.eta;
+    P.noise_mode = a.noise_mode;
+    P.noise_q2n = a.u.noise_q2n;
+    P.noise_base = a.u.noise_base;
+    P.key0 = a.key0;
+    P.key1 = a.key1;
+    P.stream = a.stream;
+    for (int i = 0; i < a.tgt[0].nterms; i++) {
+        const FusedTerm &T = a.tgt[0].term[i];
+        if (T.src != SRC_CONST || T.mult_i) return false;
+        for (int k = T.pres0; k < T.pres0 + T.npres; k++) {
+            const PresDev &D = a.pool[k];
+            if (D.q2n == 0 && D.a == 0 && D.b == 0 && D.cz == 0 && D.invq == 0) P.cst += D.c;
+        }
+    }
+    if (a.ngroups == 1) {
+        if (!lean_op(a, a.gmul[0], P.g)) return false;
+        P.nprod = a.pg0[1] - a.pg0[0];
+        if (P.nprod > LEAN_PRODS) return false;
+        for (int i = 0; i < P.nprod; i++) {
+            P.coef[i] = a.coef[a.pg0[0] + i];
+            for (int f = 0; f < a.nreal; f++) P.power[i] |= (uint32_t)a.cnt[a.pg0[0] + i][f] << (8 * f);
+        }
+    }
+    for (int f = 0; f < a.nreal; f++) {
+        LeanField &F = P.f[f];
+        if (a.zsrc[f] >= 0 || a.lbase[f] >= 0) return false;
+        P.Z[f] = a.Z[f];
+        F.lin = a.lmul[f].npres > 0;
+        if (F.lin && !lean_op(a, a.lmul[f], F.op)) return false;
+        F.kmax = a.kmax[f];
+        F.kymax = a.kymax[f];
+        F.zero = a.zero[f];
+    }
+    P.nimp = a.u.nimp;
+    double d[4] = {1.0, 0.0, 0.0, 0.0};
+    for (int i = 0; i < a.u.nimp; i++) {
+        const PresDev &D = a.u.imp[i];
+        if (D.invq != 0 || D.q2n < 0 || D.q2n > 3) return false;
+        d[D.q2n] -= (double)a.u.dt * (double)D.c;
+    }
+    for (int i = 0; i < 4; i++) P.d[i] = (float)d[i];
+    return true;
+}
+
 // device descriptor of system s (its fused plan must be ok); natural: the
 // 3D path, which needs no column-major spectra
 static int describe(cupss_system s, FusedInst &a, bool natural = false)
@@ -427,6 +504,7 @@ static int describe(cupss_system s, FusedInst &a, bool natural = false)
             a.tgt[1 + c].z = (int)i;
         }
     }
+    if (!natural) a.simple = make_lean(a) ? 1 : 0;
     if (!natural && !is_elementwise(a)) {
         if (int r = alloc_spec(&s->ft[0], g)) return r;
         if (int r = alloc_spec(&s->ft[1], g)) return r;
@@ -458,6 +536,7 @@ static bool run_view(cupss_system s, bool elementwise, FusedInst &a)
         set(a.nat, F.spec[F.cur]);
     }
     set(a.resume, !elementwise && s->resume_now ? 1 : 0);
+    a.lean.resume = a.resume;
     set(a.step_base, (uint64_t)s->step);
     set(a.cont, s->cont_now ? 1 : 0);
     const int b0 = s->cont_now ? s->cont_buf : 0;
@@ -467,7 +546,10 @@ static bool run_view(cupss_system s, bool elementwise, FusedInst &a)
         set(a.cs[c][0], s->fc[c][b0]);
         set(a.cs[c][1], s->fc[c][b0 ^ 1]);
     }
-    for (int k = 0; k < a.nreal; k++) set(a.zero[k], step0_zero(s, s->plan.real[k]) ? 1 : 0);
+    for (int k = 0; k < a.nreal; k++) {
+        set(a.zero[k], step0_zero(s, s->plan.real[k]) ? 1 : 0);
+        if (k < 2) a.lean.f[k].zero = a.zero[k];
+    }
     for (int d = 0; d < a.nder; d++) {
         FieldRec &D = s->f[s->plan.derived[d]];
         set(a.dout[d], D.spec[D.cur]);
@@ -499,6 +581,20 @@ static double inst_bytes(const FusedInst &a)
     for (int c = 0; c < a.ncons; c++)
         if (a.tgt[1 + c].noisy == NOISE_REAL) arrays++;
     return 8.0 * (double)a.g.nh * arrays;
+}
+
+// row and column launches of a size class
+static hipError_t class_rows(const FusedBatch &B, const FusedBatch::Class &c, int lpb, const Tables &t, uint32_t rel,
+                             hipStream_t st)
+{
+    return c.lean ? lean_rows_launch(c.nc, lpb, B.d, t.rb, t.nrb, rel, st)
+                  : fused_rows_launch(c.nc, lpb, c.width, B.d, t.rb, t.nrb, rel, st);
+}
+static hipError_t class_cols(const FusedBatch &B, const FusedBatch::Class &c, int twd, const Tables &t, int parity,
+                             uint32_t rel, int mode, hipStream_t st, unsigned long long *ts = nullptr)
+{
+    return c.lean ? lean_cols_launch(c.ny, twd, B.d, t.cb, t.ncb, parity, rel, mode, st, ts)
+                  : fused_cols_launch(c.ny, twd, c.cons, B.d, t.cb, t.ncb, parity, rel, mode, st, ts);
 }
 
 // row and column tables of the chunks of class c for shapes (lpb, twd)
@@ -583,7 +679,7 @@ static int build(FusedBatch &B)
         for (int k = 0; k < a.ncons; k++)
             if (a.tgt[1 + k].dyn || a.tgt[1 + k].fresh || a.tgt[1 + k].noisy) stored = 2;
         const int width = fused_row_width(a.nreal);
-        auto key = std::make_pair(a.g.nc * 16 + (width == 2 ? 0 : width == 3 ? 4 : 8) + stored, a.g.sy);
+        auto key = std::make_pair(a.g.nc * 16 + (width == 2 ? 0 : width == 3 ? 4 : 8) + (a.simple ? 3 : stored), a.g.sy);
         if (!cls.count(key)) {
             cls[key] = (int)B.classes.size();
             B.classes.emplace_back();
@@ -591,6 +687,7 @@ static int build(FusedBatch &B)
             B.classes.back().ny = a.g.sy;
             B.classes.back().width = width;
             B.classes.back().cons = stored;
+            B.classes.back().lean = a.simple != 0;
         }
         FusedBatch::Class &c = B.classes[cls[key]];
         c.insts.push_back((int)i);
@@ -685,7 +782,7 @@ static int launch_prologue(FusedBatch &B)
         for (int i : c.insts) resumed = resumed && B.h[i].resume;
         if (c.real && !resumed)
             for (auto &t : c.chunks)
-                HIP_TRY(fused_cols_launch(c.ny, c.twd, c.cons, B.d, t.cb, t.ncb, 0, 0, 0, B.stream));
+                HIP_TRY(class_cols(B, c, c.twd, t, 0, 0, 0, B.stream));
     }
     return CUPSS_OK;
 }
@@ -703,16 +800,19 @@ static int launch_class(FusedBatch &B, size_t ci, int n0, int k, int rel0, hipSt
             ts = B.pts + (size_t)(B.pcount++) * FUSED_TS_SLOTS * FUSED_TS_STRIDE;
             B.psteps = k;
         }
-        HIP_TRY(fused_small_launch(c.nc, c.ny, c.cons, B.d, c.ids, (int)c.insts.size(), n0, k, rel0, st, ts));
+        if (c.lean)
+            HIP_TRY(lean_small_launch(c.nc, c.ny, B.d, c.ids, (int)c.insts.size(), n0, k, rel0, st, ts));
+        else
+            HIP_TRY(fused_small_launch(c.nc, c.ny, c.cons, B.d, c.ids, (int)c.insts.size(), n0, k, rel0, st, ts));
         return CUPSS_OK;
     }
     for (auto &t : c.chunks)
         for (int n = n0; n < n0 + k; n++) {
-            HIP_TRY(fused_rows_launch(c.nc, c.lpb, c.width, B.d, t.rb, t.nrb, (uint32_t)(n - rel0), st));
+            HIP_TRY(class_rows(B, c, c.lpb, t, (uint32_t)(n - rel0), st));
             unsigned long long *ts = nullptr;
             if (timed && B.pcount < FusedBatch::PROF_SLOTS)
                 ts = B.pts + (size_t)(B.pcount++) * FUSED_TS_SLOTS * FUSED_TS_STRIDE;
-            HIP_TRY(fused_cols_launch(c.ny, c.twd, c.cons, B.d, t.cb, t.ncb, n & 1, (uint32_t)(n - rel0), 1, st, ts));
+            HIP_TRY(class_cols(B, c, c.twd, t, n & 1, (uint32_t)(n - rel0), 1, st, ts));
         }
     return CUPSS_OK;
 }
@@ -863,7 +963,7 @@ static int tune(FusedBatch &B)
             const int r = time_ms(
                 B, T, reps,
                 [&]() -> int {
-                    HIP_TRY(fused_rows_launch(c.nc, lpb, c.width, B.d, t[0].rb, t[0].nrb, 0, B.stream));
+                    HIP_TRY(class_rows(B, c, lpb, t[0], 0, B.stream));
                     return CUPSS_OK;
                 },
                 &ms);
@@ -886,7 +986,7 @@ static int tune(FusedBatch &B)
             const int r = time_ms(
                 B, T, reps,
                 [&]() -> int {
-                    HIP_TRY(fused_cols_launch(c.ny, twd, c.cons, B.d, t[0].cb, t[0].ncb, 0, 0, 1, B.stream));
+                    HIP_TRY(class_cols(B, c, twd, t[0], 0, 0, 1, B.stream));
                     return CUPSS_OK;
                 },
                 &ms);
@@ -1467,6 +1567,8 @@ static int kernel_time(FusedBatch &B, float *avg_ms, double *points, char *name,
         if (c.small)
             std::snprintf(name, (size_t)len, "k_fsmall<%d, %d, %s, %s>", c.nc, c.ny, c.cons ? "true" : "false",
                           c.cons == 2 ? "true" : "false");
+        else if (c.lean)
+            std::snprintf(name, (size_t)len, "k_fcols<%d, %d>", c.ny, c.twd);
         else
             std::snprintf(name, (size_t)len, "k_fcols<%d, %d, %s, %s>", c.ny, c.twd, c.cons ? "true" : "false",
                           c.cons == 2 ? "true" : "false");

@@ -88,7 +88,7 @@ __global__ __launch_bounds__((FColCfg<N, TWD>::THREADS)) void k_fcols(const Fuse
 
 // ------------------------------------------------------------ small instances
 
-// Instances small enough for one workgroup (64^2, 128^2): K steps in one
+// Instances small enough for one workgroup (64^2): K steps in one
 // launch, one workgroup per instance, each step the same row and column
 // tiles as the two-kernel step (so the same results bit for bit) in turn,
 // separated by workgroup barriers -- no launch per pass, and the
@@ -825,10 +825,14 @@ hipError_t fused_cols_launch(int ny, int twd, int stored, const FusedInst *inst,
     }
 }
 
-bool fused_small_class(int nc, int ny, int width)
-{
-    return width <= 3 && ny == 2 * nc && (ny == 64 || ny == 128);
-}
+// 64^2: one workgroup takes the steps in one launch, without a kernel boundary
+// per pass; on 128^2 one CU's vector issue is the bound and two launches per
+// step over the chip are faster.  us per step, one workgroup / two launches:
+// CH 64^2 5.9 / 8.2, KPZ 64^2 11.8 / 12.9, Gray-Scott 64^2 16.6 / 18.0; KPZ
+// 128^2 42 / 16, Gray-Scott 128^2 48 / 21.  Many instances at once hide either
+// (512 EW/KPZ instances: 169 us per step with 128^2 on one workgroup each or
+// not).
+bool fused_small_class(int nc, int ny, int width) { return width <= 3 && nc == 32 && ny == 64; }
 
 template <int NC, int N>
 static hipError_t fsmall_n(int stored, const FusedInst *inst, const int *ids, int nids, int n0, int k, int rel0,
@@ -856,7 +860,6 @@ hipError_t fused_small_launch(int nc, int ny, int stored, const FusedInst *inst,
     if (!sets) return hipErrorOutOfMemory;
     if (nids <= 0 || k <= 0) return hipSuccess;
     if (nc == 32 && ny == 64) return fsmall_n<32, 64>(stored, inst, ids, nids, n0, k, rel0, s, sets, ts);
-    if (nc == 64 && ny == 128) return fsmall_n<64, 128>(stored, inst, ids, nids, n0, k, rel0, s, sets, ts);
     return hipErrorInvalidValue;
 }
 

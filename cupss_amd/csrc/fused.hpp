@@ -82,6 +82,39 @@ struct FusedTarget {
     float2 *eta;     // NOISE_REAL: R2C_x(xi) rows, column-major (row pass)
 };
 
+// The program of a simple system in 256 bytes that a workgroup loads at once
+// (lean_tiles.hpp): phi alone (no stored fields; its other terms are
+// constants), at most one product group and two real fields that are phi or
+// monomials of it, a polynomial implicit operator.
+constexpr int LEAN_PRODS = 4;
+struct LeanOp {                   // c q^(2 q2n) (i qx)^a (i qy)^b with the sign folded into c
+    float c;
+    int q2n, a, b, mult_i;
+};
+struct LeanField {
+    LeanOp op;
+    int lin;                      // 0: the field is phi itself
+    int kmax, kymax, zero;        // as FusedInst
+};
+struct alignas(64) FusedLean {
+    float2 *X, *Z[2], *eta;
+    int sy, nc, nc1;
+    float sqx, sqy;
+    float scale, dt;
+    int nreal, ngroups, nprod;
+    int noise_mode, noise_q2n;
+    float noise_base;
+    uint32_t key0, key1, stream;
+    float coef[LEAN_PRODS];
+    uint32_t power[LEAN_PRODS];   // of field 0 (bits 0-7) and field 1 (bits 8-15)
+    LeanOp g;                     // the group's multiplier
+    float cst;                    // constant terms: their sum at q = 0
+    int nimp;
+    float d[4];                   // D(q) = sum_n d[n] q^(2n)
+    int resume;
+    LeanField f[2];
+};
+
 // Device-side descriptor of one instance (one system) of a fused batch.
 //
 // Transform instances keep phi's spectrum and every pipeline buffer
@@ -89,6 +122,8 @@ struct FusedTarget {
 // kernel reads and writes whole contiguous columns.  Elementwise instances
 // use the natural half-spectrum layout (ky, kx) of the system buffers.
 struct FusedInst {
+    FusedLean lean;
+    int simple;                               // lean holds the system
     Geom g;
     float2 *spec[2];                          // phi's spectrum: [parity] in, [parity^1] out
     float2 *nat;                              // the system's spectrum (natural layout), transform instances
@@ -163,13 +198,21 @@ hipError_t fused_rows_launch(int nc, int lpb, int width, const FusedInst *inst, 
 // constraints)
 hipError_t fused_cols_launch(int ny, int twd, int stored, const FusedInst *inst, const FusedBlock *blocks, int nblocks,
                              int parity, uint32_t step_rel, int mode, hipStream_t s, unsigned long long *ts = nullptr);
-// Size classes whose instances take whole steps in one workgroup each
-// (64^2, 128^2): k steps [n0, n0+k) of the instances ids[0..nids) in one
+// the same for launches whose instances are all simple (FusedInst::simple):
+// row shapes of width 2
+hipError_t lean_rows_launch(int nc, int lpb, const FusedInst *inst, const FusedBlock *blocks, int nblocks,
+                            uint32_t step_rel, hipStream_t s);
+hipError_t lean_cols_launch(int ny, int twd, const FusedInst *inst, const FusedBlock *blocks, int nblocks, int parity,
+                            uint32_t step_rel, int mode, hipStream_t s, unsigned long long *ts = nullptr);
+// Size class whose instances take whole steps in one workgroup each (64^2):
+// k steps [n0, n0+k) of the instances ids[0..nids) in one
 // launch (step n reads spectrum buffer n&1, noise counter offset n - rel0);
 // stored and ts as for fused_cols_launch (one slot pair for the launch).
 bool fused_small_class(int nc, int ny, int width);
 hipError_t fused_small_launch(int nc, int ny, int stored, const FusedInst *inst, const int *ids, int nids, int n0,
                               int k, int rel0, hipStream_t s, unsigned long long *ts = nullptr);
+hipError_t lean_small_launch(int nc, int ny, const FusedInst *inst, const int *ids, int nids, int n0, int k, int rel0,
+                             hipStream_t s, unsigned long long *ts = nullptr);
 // the slots of n timed launches to {~0, 0} (a kernel, so that graphs can hold it)
 hipError_t fused_ts_reset_launch(unsigned long long *ts, int n, hipStream_t s);
 // ---- 3D systems (one instance, natural half-spectrum layout; insts[0]).
