@@ -380,7 +380,6 @@ static int describe(cupss_system s, FusedInst &a, bool natural = false)
     int np = 0;
     auto index_of = [](const std::vector<int> &v, int x) { return (int)(std::find(v.begin(), v.end(), x) - v.begin()); };
     // derived fields: one multiplier each (also L_f of their real fields)
-    if (!fused_noise_ok(s)) return fail(CUPSS_ERR_UNSUPPORTED, "the fused 3D step draws noise in spectral space only");
     a.nder = (int)P.derived.size();
     for (size_t d = 0; d < P.derived.size(); d++) {
         if (int r = pool_term(a, np, s->t[s->f[P.derived[d]].terms[0]].pres, a.dmul[d])) return r;
@@ -1229,9 +1228,9 @@ static int tune3d(FusedBatch &B, cupss_system s, int par, uint32_t rel)
     int rc = CUPSS_OK;
     for (int w : v) {
         float ms = 0;
-        hipError_t e = fused3d_z_launch(g.sz, w, B.d, g.nc1, g.sy, par, rel, 2, st);  // warm-up
+        hipError_t e = fused3d_z_launch(g.sz, w, B.d, g.nc1, g.sy, par, rel, 2, 0, st);  // warm-up
         if (e == hipSuccess) e = hipEventRecord(e0, st);
-        for (int r = 0; r < 3 && e == hipSuccess; r++) e = fused3d_z_launch(g.sz, w, B.d, g.nc1, g.sy, par, rel, 2, st);
+        for (int r = 0; r < 3 && e == hipSuccess; r++) e = fused3d_z_launch(g.sz, w, B.d, g.nc1, g.sy, par, rel, 2, 0, st);
         if (e == hipSuccess) e = hipEventRecord(e1, st);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
         if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
@@ -1250,14 +1249,14 @@ static int tune3d(FusedBatch &B, cupss_system s, int par, uint32_t rel)
     return rc;
 }
 
-// The fused step of a 3D system (fused.hip: k_f3rows, k_f3z; the y lines
-// by lines_y), natural layout, no transposes.  A run is
+// The fused step of a 3D system (fused3d.hip), natural layout, no transposes.  A run is
 //   prologue:  z pass in mode 0 and IFFT_y: W_f, Z_f of the current state
 //              (skipped when the previous run left them and nothing changed
 //              the system since: per-step callers pay no prologue);
-//   steps:     rows, FFT_y of every group, z pass (update; W_f of the new
-//              state), IFFT_y of every real field;
-//   end:       the derived fields of the last step's starting phi.
+//   steps:     rows, FFT_y of every group and of the noise, z pass (update;
+//              W_f of the new state), IFFT_y of every real field;
+//   end:       the Hermitian projection of the final state, the derived
+//              fields of the last step's starting phi.
 // The descriptor keeps both spectrum buffers of phi in a fixed order (the
 // launches pass the parity) and is uploaded again only when it changes.
 static int run3d(FusedBatch &B, cupss_system s, int nsteps)
@@ -1309,19 +1308,41 @@ static int run3d(FusedBatch &B, cupss_system s, int nsteps)
         B.h.assign(1, a);
         B.d3 = true;
     }
-    if (!twiddle_sets(s->stream) || !twiddles(s->stream)) return fail(CUPSS_ERR_NOMEM, "twiddle tables");
+    if (!twiddle_sets(s->stream)) return fail(CUPSS_ERR_NOMEM, "twiddle tables");
     const uint32_t rel0 = (uint32_t)(s->step - B.h[0].step_base);
-    const int par0 = F.cur, maxr = a.nreal > 3 ? FUSED_MAX_REAL : 3;
+    const int par0 = F.cur, maxr = a.nreal > 3 ? FUSED_MAX_REAL : (a.nreal > 1 ? 3 : 1);
     const long nrows = (long)g.sy * g.sz;
     hipStream_t st = s->stream;
     if (!B.twd3)
         if (int r = tune3d(B, s, par0, rel0)) return r;
+    // the y passes: all products and the noise, all real fields
+    const float2 *fin[FUSED_MAX_GROUPS + 1];
+    float2 *fout[FUSED_MAX_GROUPS + 1];
+    int fcols[FUSED_MAX_GROUPS + 1], nf = 0;
+    auto forward = [&](float2 *x) {
+        fin[nf] = x;
+        fout[nf] = x;
+        fcols[nf++] = g.nc1;
+    };
+    for (int gi = 0; gi < a.ngroups; gi++) forward(s->fx[gi]);
+    if (a.noise_mode == NOISE_REAL) forward(F.eta);
+    auto inverse_y = [&]() {
+        const float2 *in[FUSED_MAX_REAL];
+        float2 *out[FUSED_MAX_REAL];
+        int cols[FUSED_MAX_REAL];
+        for (int f = 0; f < a.nreal; f++) {
+            in[f] = s->fw[f];
+            out[f] = s->fz[f];
+            cols[f] = a.kmax[f] + 1;
+        }
+        return fused3d_y_launch(g, +1, a.nreal, in, out, cols, st);
+    };
     // Z_f of the current state: left by the previous run when nothing changed
     // the system since (each run ends with them), else the prologue
     const bool cont = s->cont_step == s->step && s->cont_gen == s->gen;
     if (a.nreal > 0 && !cont) {
-        HIP_TRY(fused3d_z_launch(g.sz, B.twd3, B.d, g.nc1, g.sy, par0, rel0, 0, st));
-        for (int f = 0; f < a.nreal; f++) HIP_TRY(lines_y(g, +1, s->fw[f], s->fz[f], a.kmax[f] + 1, st));
+        HIP_TRY(fused3d_z_launch(g.sz, B.twd3, B.d, g.nc1, g.sy, par0, rel0, 0, 0, st));
+        HIP_TRY(inverse_y());
     }
     if (B.profile) {
         B.pclass = -2;
@@ -1329,18 +1350,20 @@ static int run3d(FusedBatch &B, cupss_system s, int nsteps)
         HIP_TRY(fused_ts_reset_launch(B.pts, FusedBatch::PROF_SLOTS, st));
     }
     for (int i = 0; i < nsteps; i++) {
-        if (a.ngroups > 0) {
-            HIP_TRY(fused3d_rows_launch(g.nc, maxr, B.d, nrows, st));
-            for (int gi = 0; gi < a.ngroups; gi++) HIP_TRY(lines_y(g, -1, s->fx[gi], s->fx[gi], g.nc1, st));
+        if (nf > 0) {
+            HIP_TRY(fused3d_rows_launch(g.nc, maxr, B.d, nrows, rel0 + (uint32_t)i, st));
+            HIP_TRY(fused3d_y_launch(g, -1, nf, fin, fout, fcols, st));
         }
         unsigned long long *ts = nullptr;
         if (B.profile && B.pcount < FusedBatch::PROF_SLOTS)
             ts = B.pts + (size_t)(B.pcount++) * FUSED_TS_SLOTS * FUSED_TS_STRIDE;
-        HIP_TRY(fused3d_z_launch(g.sz, B.twd3, B.d, g.nc1, g.sy, par0 ^ (i & 1), rel0 + (uint32_t)i, 1, st, ts));
-        // the kx = 0, sx/2 planes of the new state: partners are in other z lines
-        HIP_TRY(hermitian_planes(g, F.spec[par0 ^ (i & 1) ^ 1], st));
-        for (int f = 0; f < a.nreal; f++) HIP_TRY(lines_y(g, +1, s->fw[f], s->fz[f], a.kmax[f] + 1, st));
+        HIP_TRY(fused3d_z_launch(g.sz, B.twd3, B.d, g.nc1, g.sy, par0 ^ (i & 1), rel0 + (uint32_t)i, 1, i > 0, st, ts));
+        HIP_TRY(inverse_y());
     }
+    // the kx = 0, sx/2 planes of the final state (partners are in other z
+    // lines; the steps before project their predecessor's on reading)
+    HIP_TRY(hermitian_planes(g, F.spec[par0 ^ (nsteps & 1)], st));
+    if (a.nder > 0 && nsteps > 1) HIP_TRY(hermitian_planes(g, F.spec[par0 ^ ((nsteps - 1) & 1)], st));
     if (a.nder > 0) HIP_TRY(fused3d_derived_launch(B.d, g.nh, par0 ^ ((nsteps - 1) & 1), st));
     F.cur = par0 ^ (nsteps & 1);
     s->step += (uint64_t)nsteps;

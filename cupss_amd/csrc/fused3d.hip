@@ -2,6 +2,8 @@
 // field (the systems and descriptors are those of fused.hip).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "fft_core.hpp"
 #include "fused.hpp"
 #include "fused_tiles.hpp"
@@ -16,22 +18,25 @@ namespace cupss {
 // spectrum layout, element (kx, ky, kz) at (kz*sy + ky)*nc1 + kx, so no
 // transposes are needed: rows are contiguous, and lines along y and z are
 // read TWD adjacent kx at a time.  Per step:
-//   rows  (k_f3rows): Z_f rows -C2R_x-> real fields -> products -R2C_x-> X_g
-//   y     (lines_y):  X_g = FFT_y(X_g)
-//   z     (k_f3z):    X_g -FFT_z-> terms; update of phi (setDynamic_k);
-//                     mask_f * L_f * phi_new -IFFT_z-> W_f
-//   y     (lines_y):  Z_f = IFFT_y(W_f), lines kx <= kmax_f
+//   rows  (k_f3rows): Z_f rows -C2R_x-> real fields -> products -R2C_x-> X_g;
+//                     real-space noise -R2C_x-> eta
+//   y     (k_f3y):    X_g = FFT_y(X_g), eta = FFT_y(eta), in one launch
+//   z     (k_f3z):    X_g, eta -FFT_z-> terms, noise; update of phi
+//                     (setDynamic_k); mask_f * L_f * phi_new -IFFT_z-> W_f
+//   y     (k_f3y):    Z_f = IFFT_y(W_f), lines kx <= kmax_f, in one launch
 // W_f is written only on the (kx, ky) lines the dealias mask of f keeps; the
 // others stay zero from allocation.  The systems have no stored constraint
-// fields and no real-space noise (the host checks).
+// fields (the host checks).
 
 template <int NC, int LPB, int MAXR>
 __global__ __launch_bounds__((FRowCfg<NC, LPB, MAXR>::THREADS)) void k_f3rows(const FusedInst *__restrict__ insts,
+                                                                           uint32_t step_rel,
                                                                            const float2 *__restrict__ sets)
 {
     using C = FRowCfg<NC, LPB, MAXR>;
     constexpr int E = C::E, T = C::T, RS = C::RS;
     __shared__ float2 tws[2 * NC];
+    __shared__ __align__(16) float2 tst[tw_stage_alloc(NC, E)];
     __shared__ float2 tile[LPB * RS];
     const FusedInst &a = insts[0];
     const int nc1 = a.g.nc1;
@@ -42,6 +47,7 @@ __global__ __launch_bounds__((FRowCfg<NC, LPB, MAXR>::THREADS)) void k_f3rows(co
     float2 *L = tile + l * RS;
     const int nreal = a.nreal;
     load_twiddles<2 * NC>(tws, sets);
+    load_stage_twiddles<NC, E>(tst, sets);
     __syncthreads();
 
     float2 r[MAXR][E];
@@ -58,7 +64,7 @@ __global__ __launch_bounds__((FRowCfg<NC, LPB, MAXR>::THREADS)) void k_f3rows(co
                 ya[e] = (active && NC - k <= km) ? gload(z, NC - k) : make_float2(0.f, 0.f);
             }
             c2r_prep<NC, E, T>(xa, ya, t, v, tws);
-            fft_line<NC, E, +1, 2 * NC, false, (T <= 64)>(v, L, t, tws);
+            fft_line<NC, E, +1, TW_STAGE, false, (T <= 64)>(v, L, t, tst);
 #pragma unroll
             for (int e = 0; e < E; e++) r[f][e] = cscale(v[e], a.scale);
             line_sync<(T <= 64)>();
@@ -85,13 +91,91 @@ __global__ __launch_bounds__((FRowCfg<NC, LPB, MAXR>::THREADS)) void k_f3rows(co
 #pragma unroll
             for (int e = 0; e < E; e++) v[e] = cadd(v[e], p[e]);
         }
-        r2c_tile<NC, E, T, 2 * NC>(v, L, t, tws, tws);
+        r2c_tile<NC, E, T, TW_STAGE>(v, L, t, tws, tst);
         if (active) {
             float2 *__restrict__ x = a.X[gi] + row * nc1;
             for (int k = t; k <= NC; k += T) gstore(x, k, L[k]);
         }
         __syncthreads();
     }
+    if (a.noise_mode == NOISE_REAL) {
+        // cells 2k, 2k+1 of the row, k = t + e*T: lanes t, t^1 share Philox
+        // calls and swap the pairs (frows_tile)
+        const uint64_t step = a.step_base + step_rel;
+        const uint32_t rowbase = (uint32_t)(row * NC);
+        const bool even = (t & 1) == 0;
+        float2 v[E];
+#pragma unroll
+        for (int e2 = 0; e2 < E / 2; e2++) {
+            const uint32_t k = (uint32_t)((t & ~1) + (even ? e2 : e2 + E / 2) * T);
+            const Philox4 o = philox4x32_10((rowbase + k) >> 1, (uint32_t)step, (uint32_t)(step >> 32), a.stream,
+                                            a.key0, a.key1);
+            const float2 ze = box_muller(o.x[0], o.x[1]), zo = box_muller(o.x[2], o.x[3]);
+            const float2 own = even ? ze : zo, snd = even ? zo : ze;
+            const float2 rcv = make_float2(__shfl_xor(snd.x, 1), __shfl_xor(snd.y, 1));
+            v[e2] = even ? own : rcv;
+            v[e2 + E / 2] = even ? rcv : own;
+        }
+        r2c_tile<NC, E, T, TW_STAGE>(v, L, t, tws, tst);
+        if (active) {
+            float2 *__restrict__ x = a.eta + row * nc1;
+            for (int k = t; k <= NC; k += T) gstore(x, k, L[k]);
+        }
+    }
+}
+
+// Lines along y of several buffers at once (blockIdx.y: the buffer): line
+// (kx, kz) of a buffer holds in[(kz*sy + y)*nc1 + kx], kx < ncols; TWD
+// adjacent kx per workgroup, out may be in.  Bound by memory on large boxes
+// (256^3, one buffer forward: 134 MB in 23 us, 5.8 TB/s), by latency on small
+// ones, where one launch for all buffers fills the chip: 128^3 with noise,
+// the two forward transforms 16.4 us in two launches of the general column
+// kernel, 8.8 us here.
+constexpr int F3Y_BUFS = FUSED_MAX_GROUPS + 1;
+struct F3yArgs {
+    const float2 *in[F3Y_BUFS];
+    float2 *out[F3Y_BUFS];
+    int ncols[F3Y_BUFS];
+    int nc1, sz;
+};
+template <int N, int TWD>
+struct F3yCfg {
+    static constexpr int E = N >= 4096 ? 16 : (N >= 8 ? 8 : N);
+    static constexpr int T = N / E;
+    static constexpr int THREADS = TWD * T;
+    static constexpr int LL = lds_len(N);
+    static constexpr bool valid() { return THREADS >= 64 && THREADS <= 512; }
+};
+template <int N, int TWD, int DIR>
+__global__ __launch_bounds__((F3yCfg<N, TWD>::THREADS)) void k_f3y(F3yArgs a, const float2 *__restrict__ sets)
+{
+    using C = F3yCfg<N, TWD>;
+    constexpr int E = C::E, T = C::T;
+    constexpr bool WL = TWD * T <= 64;
+    __shared__ __align__(16) float2 tst[tw_stage_alloc(N, E)];
+    __shared__ float2 lds[TWD * C::LL];
+    const int nc1 = a.nc1, ncols = a.ncols[blockIdx.y];
+    const int ntx = (ncols + TWD - 1) / TWD;
+    const long item = xcd_item(blockIdx.x, gridDim.x);
+    if (item >= (long)ntx * a.sz) return;  // whole workgroup idle
+    const int kz = (int)(item / ntx), kx0 = (int)(item % ntx) * TWD;
+    const int c = threadIdx.x % TWD, t = threadIdx.x / TWD;
+    const bool active = kx0 + c < ncols;
+    const long base = (long)kz * N * nc1 + kx0 + c;
+    StageTwiddles<N, E, C::THREADS> twl;
+    twl.load(sets);
+    const float2 *in = a.in[blockIdx.y];
+    float2 v[E];
+#pragma unroll
+    for (int e = 0; e < E; e++)
+        v[e] = active ? gload(in, base + (long)(t + e * T) * nc1) : make_float2(0.f, 0.f);
+    twl.store(tst, sets);
+    __syncthreads();
+    fft_line<N, E, DIR, TW_STAGE, false, WL>(v, lds + c * C::LL, t, tst);
+    if (!active) return;
+    float2 *out = a.out[blockIdx.y];
+#pragma unroll
+    for (int e = 0; e < E; e++) gstore(out, base + (long)(t + e * T) * nc1, v[e]);
 }
 
 // q of the E bins (kx, ky, t + e*T) that one lane of a z-line kernel holds
@@ -162,13 +246,13 @@ struct F3zCfg {
 // strided HBM accesses, which more resident waves hide.
 template <int N, int TWD>
 __global__ __launch_bounds__((F3zCfg<N, TWD>::THREADS)) __attribute__((amdgpu_waves_per_eu(4))) void k_f3z(const FusedInst *__restrict__ insts, int parity,
-                                                                 uint32_t step_rel, int mode,
+                                                                 uint32_t step_rel, int mode, int herm,
                                                                  const float2 *__restrict__ sets,
                                                                  unsigned long long *__restrict__ ts)
 {
     using C = F3zCfg<N, TWD>;
     constexpr int E = C::E, T = C::T;
-    __shared__ float2 tws[N];
+    __shared__ __align__(16) float2 tws[tw_stage_alloc(N, E)];
     __shared__ float2 lds[TWD * C::LL];
     const FusedInst &a = insts[0];
     const Geom &g = a.g;
@@ -199,7 +283,21 @@ __global__ __launch_bounds__((F3zCfg<N, TWD>::THREADS)) __attribute__((amdgpu_wa
         cur[e] = active ? gload(sin, i) : make_float2(0.f, 0.f);
         xv[e] = (active && upd && TG.g1 > TG.g0) ? gload(a.X[TG.g0], i) : make_float2(0.f, 0.f);
     }
-    load_twiddles<N>(tws, sets);
+    if (herm && (kx0 == 0 || kx0 + TWD > g.nc)) {
+        // The previous step of this launch sequence left the kx = 0 and sx/2
+        // planes as it computed them: their Hermitian projection
+        // (k_hermitian_planes, the last step's is done by it) as they are
+        // read, bin (ky, kz) with its partner (-ky, -kz)
+        if (kx == 0 || kx == g.nc) {
+            const long pbase = (long)((g.sy - ky) & (g.sy - 1)) * g.nc1 + kx;
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                const float2 p = gload(sin, pbase + (long)((N - (t + e * T)) & (N - 1)) * plane);
+                cur[e] = make_float2(0.5f * (cur[e].x + p.x), 0.5f * (cur[e].y - p.y));
+            }
+        }
+    }
+    load_stage_twiddles<N, E>(tws, sets);
     __syncthreads();
 
     LineBins<E> lb;
@@ -217,7 +315,7 @@ __global__ __launch_bounds__((F3zCfg<N, TWD>::THREADS)) __attribute__((amdgpu_wa
                 for (int e = 0; e < E; e++)
                     xv[e] = active ? gload(a.X[gi], base + (long)(t + e * T) * plane) : make_float2(0.f, 0.f);
             }
-            fft_line<N, E, -1, N, true, (TWD * T <= 64)>(xv, L, t, tws);
+            fft_line<N, E, -1, TW_STAGE, false, (TWD * T <= 64)>(xv, L, t, tws);
             const TermRefDev &GM = a.gmul[gi];
             multiplier_line<E>(a.pool, GM.pres0, GM.npres, GM.mult_i, lb, m);
 #pragma unroll
@@ -247,15 +345,24 @@ __global__ __launch_bounds__((F3zCfg<N, TWD>::THREADS)) __attribute__((amdgpu_wa
         }
         const UpdateArgs &u = a.u;
         const uint64_t step = a.step_base + step_rel;
+        const bool real_noise = u.noisy && a.noise_mode == NOISE_REAL;
+        if (real_noise) {
+#pragma unroll
+            for (int e = 0; e < E; e++)
+                xv[e] = active ? gload(a.eta, base + (long)(t + e * T) * plane) : make_float2(0.f, 0.f);
+            fft_line<N, E, -1, TW_STAGE, false, (TWD * T <= 64)>(xv, L, t, tws);
+            line_sync<(TWD * T <= 64)>();
+        }
 #pragma unroll
         for (int e = 0; e < E; e++) {
             float2 s = cur[e];
             s.x += u.dt * acc[e].x;
             s.y += u.dt * acc[e].y;
-            if (u.noisy && a.noise_mode == NOISE_SPECTRAL) {
-                const float2 eta = active ? spectral_noise(g, kx, ky, t + e * T, (uint32_t)step, (uint32_t)(step >> 32),
-                                                           a.stream, a.key0, a.key1)
-                                          : make_float2(0.f, 0.f);
+            if (u.noisy) {
+                const float2 eta = real_noise ? xv[e]
+                                   : active   ? spectral_noise(g, kx, ky, t + e * T, (uint32_t)step,
+                                                               (uint32_t)(step >> 32), a.stream, a.key0, a.key1)
+                                              : make_float2(0.f, 0.f);
                 float pn = u.noise_base;
                 if (u.noise_q2n != 0) pn *= sqrtf(ipow(lb.q2[e], u.noise_q2n));
                 if (u.noise_invq != 0)
@@ -306,7 +413,7 @@ __global__ __launch_bounds__((F3zCfg<N, TWD>::THREADS)) __attribute__((amdgpu_wa
                 const float2 w = LM.npres > 0 ? apply_mult(lm[e], LM.mult_i, nw[e]) : nw[e];
                 v[e] = keep ? w : make_float2(0.f, 0.f);
             }
-            fft_line<N, E, +1, N, true, (TWD * T <= 64)>(v, L, t, tws);
+            fft_line<N, E, +1, TW_STAGE, false, (TWD * T <= 64)>(v, L, t, tws);
             if (active && kx <= a.kmax[f]) {
                 float2 *__restrict__ w = a.W[f];
 #pragma unroll
@@ -344,17 +451,17 @@ __global__ __launch_bounds__(256) void k_f3der(const FusedInst *__restrict__ ins
 #define FUSED_WIDE_NC(NC) ((NC) >= 32 && (NC) <= 1024)
 
 template <int NC, int MAXR>
-static hipError_t f3rows_n(const FusedInst *inst, long nrows, hipStream_t s, const float2 *sets)
+static hipError_t f3rows_n(const FusedInst *inst, long nrows, uint32_t step_rel, hipStream_t s, const float2 *sets)
 {
     constexpr int T = FRowCfg<NC, 1, MAXR>::T;
     constexpr int LPB = T >= 256 ? 1 : 256 / T;  // 256 threads a workgroup
     static_assert(FRowCfg<NC, LPB, MAXR>::valid(), "3D row tile");
     hipLaunchKernelGGL((k_f3rows<NC, LPB, MAXR>), dim3((unsigned)((nrows + LPB - 1) / LPB)),
-                       dim3(FRowCfg<NC, LPB, MAXR>::THREADS), 0, s, inst, sets);
+                       dim3(FRowCfg<NC, LPB, MAXR>::THREADS), 0, s, inst, step_rel, sets);
     return hipGetLastError();
 }
 
-hipError_t fused3d_rows_launch(int nc, int maxr, const FusedInst *inst, long nrows, hipStream_t s)
+hipError_t fused3d_rows_launch(int nc, int maxr, const FusedInst *inst, long nrows, uint32_t step_rel, hipStream_t s)
 {
     const float2 *sets = twiddle_sets(s);
     if (!sets) return hipErrorOutOfMemory;
@@ -363,11 +470,70 @@ hipError_t fused3d_rows_launch(int nc, int maxr, const FusedInst *inst, long nro
     case NC:                                                                  \
         if (maxr > 3) {                                                       \
             if constexpr (FUSED_WIDE_NC(NC))                                  \
-                return f3rows_n<NC, FUSED_MAX_REAL>(inst, nrows, s, sets);    \
+                return f3rows_n<NC, FUSED_MAX_REAL>(inst, nrows, step_rel, s, sets); \
             return hipErrorInvalidValue;                                      \
         }                                                                     \
-        return f3rows_n<NC, 3>(inst, nrows, s, sets);
+        if (maxr == 1) return f3rows_n<NC, 1>(inst, nrows, step_rel, s, sets); \
+        return f3rows_n<NC, 3>(inst, nrows, step_rel, s, sets);
         X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
+#undef X
+    default:
+        return hipErrorInvalidValue;
+    }
+}
+
+#define F3Y_CASES(X) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096)
+#define F3Y_TWD(X) X(1) X(2) X(4) X(8) X(16) X(32) X(64)
+
+template <int N>
+static hipError_t f3y_n(int dir, const F3yArgs &a, int nbuf, hipStream_t s, const float2 *sets)
+{
+    int most = 1;
+    for (int b = 0; b < nbuf; b++) most = std::max(most, a.ncols[b]);
+    // 16 adjacent lines (128 bytes a row, one cache line) where that still
+    // gives two workgroups a CU, else narrower: 128^3, two buffers, 16 lines
+    // 8.8 us against 16.4 us for 4 lines of a buffer at a time
+    int pick = 0;
+#define X(TWD)                                                                                              \
+    if constexpr (F3yCfg<N, TWD>::valid())                                                                  \
+        if (!pick || (TWD <= 16 && (long)((most + TWD - 1) / TWD) * a.sz * nbuf >= 512)) pick = TWD;
+    F3Y_TWD(X)
+#undef X
+#define X(TWD)                                                                                              \
+    if constexpr (F3yCfg<N, TWD>::valid())                                                                  \
+        if (pick == TWD) {                                                                                  \
+            const dim3 grid((unsigned)xcd_blocks((long)((most + TWD - 1) / TWD) * a.sz), (unsigned)nbuf);   \
+            if (dir < 0)                                                                                    \
+                hipLaunchKernelGGL((k_f3y<N, TWD, -1>), grid, dim3(F3yCfg<N, TWD>::THREADS), 0, s, a, sets); \
+            else                                                                                            \
+                hipLaunchKernelGGL((k_f3y<N, TWD, +1>), grid, dim3(F3yCfg<N, TWD>::THREADS), 0, s, a, sets); \
+            return hipGetLastError();                                                                       \
+        }
+    F3Y_TWD(X)
+#undef X
+    return hipErrorInvalidValue;
+}
+
+hipError_t fused3d_y_launch(const Geom &g, int dir, int nbuf, const float2 *const *in, float2 *const *out,
+                            const int *ncols, hipStream_t s)
+{
+    const float2 *sets = twiddle_sets(s);
+    if (!sets) return hipErrorOutOfMemory;
+    if (nbuf <= 0) return hipSuccess;
+    if (nbuf > F3Y_BUFS) return hipErrorInvalidValue;
+    F3yArgs a{};
+    for (int b = 0; b < nbuf; b++) {
+        a.in[b] = in[b];
+        a.out[b] = out[b];
+        a.ncols[b] = ncols[b];
+    }
+    a.nc1 = g.nc1;
+    a.sz = g.sz;
+    switch (g.sy) {
+#define X(N) \
+    case N:  \
+        return f3y_n<N>(dir, a, nbuf, s, sets);
+        F3Y_CASES(X)
 #undef X
     default:
         return hipErrorInvalidValue;
@@ -403,14 +569,14 @@ std::vector<int> fused3d_z_shapes(int nz)
 
 template <int N>
 static hipError_t f3z_n(int twd, const FusedInst *inst, int nc1, int sy, int parity, uint32_t step_rel, int mode,
-                        hipStream_t s, const float2 *sets, unsigned long long *ts)
+                        int herm, hipStream_t s, const float2 *sets, unsigned long long *ts)
 {
 #define X(TWD)                                                                                           \
     if constexpr (F3zCfg<N, TWD>::valid()) {                                                            \
         if (twd == TWD) {                                                                                \
             const long total = (long)((nc1 + TWD - 1) / TWD) * sy;                                       \
             hipLaunchKernelGGL((k_f3z<N, TWD>), dim3((unsigned)xcd_blocks(total)),                      \
-                               dim3(F3zCfg<N, TWD>::THREADS), 0, s, inst, parity, step_rel, mode, sets, ts); \
+                               dim3(F3zCfg<N, TWD>::THREADS), 0, s, inst, parity, step_rel, mode, herm, sets, ts); \
             return hipGetLastError();                                                                    \
         }                                                                                                \
     }
@@ -420,14 +586,14 @@ static hipError_t f3z_n(int twd, const FusedInst *inst, int nc1, int sy, int par
 }
 
 hipError_t fused3d_z_launch(int nz, int twd, const FusedInst *inst, int nc1, int sy, int parity, uint32_t step_rel,
-                            int mode, hipStream_t s, unsigned long long *ts)
+                            int mode, int herm, hipStream_t s, unsigned long long *ts)
 {
     const float2 *sets = twiddle_sets(s);
     if (!sets) return hipErrorOutOfMemory;
     switch (nz) {
 #define X(N) \
     case N:  \
-        return f3z_n<N>(twd, inst, nc1, sy, parity, step_rel, mode, s, sets, ts);
+        return f3z_n<N>(twd, inst, nc1, sy, parity, step_rel, mode, herm, s, sets, ts);
         F3Z_CASES(X)
 #undef X
     default:

@@ -106,10 +106,6 @@ hipError_t update(const UpdateArgs &a, hipStream_t s);
 // bins (kx, ky, kz), (kx, -ky, -kz) of the planes kx = 0, sx/2 -> their
 // Hermitian mean, in place
 hipError_t hermitian_planes(const Geom &g, float2 *spec, hipStream_t s);
-// unnormalised C2C transforms (dir -1 forward, +1 inverse) of the lines along
-// y of a natural half spectrum with kx < ncols: line (kx, kz) holds
-// in[(kz*sy + ky)*nc1 + kx], ky < sy; out may be in
-hipError_t lines_y(const Geom &g, int dir, const float2 *in, float2 *out, long ncols, hipStream_t s);
 // eta_hat with the law of R2C(xi), xi ~ N(0,1) per cell, from Philox
 hipError_t spectral_noise_fill(const Geom &g, float2 *eta, uint64_t seed, uint64_t step, uint32_t stream,
                                hipStream_t s);

@@ -158,7 +158,7 @@ int cupss_system_set_stream(cupss_system s, void *hip_stream);
  * linear in one of them, constraint fields of products (of dynamic fields,
  * or of derived and other such constraint fields) and coefficient fields
  * without terms; the fused 3D step takes one dynamic field with fields
- * linear in it and spectral-space noise.  Neither takes field callbacks
+ * linear in it and noise of either draw (real-space from 32^3 points).  Neither takes field callbacks
  * (either kind) or grids outside 16..4096 x 8..4096 (x 8..1024).  1D systems
  * without callbacks run the general program's steps in one workgroup, any
  * number per launch, where their fields fit its LDS. */
