@@ -15,8 +15,21 @@ namespace cupss {
 
 // MAXR: real fields a row holds at once (2, 3, or FUSED_MAX_REAL for systems
 // with more; those use 4 elements per lane to stay within the registers).
-// Rows of 1024 real points also take 4 per lane (more waves for one large
-// system).
+//
+// Elements per lane (E) of rows and columns.  On a small grid a wavefront is
+// alone on its SIMD and bound by the issue of its own instructions: fewer
+// elements a lane, that is more wavefronts, are faster as long as a line
+// stays inside one wavefront.  Many instances at once prefer fewer exchanges.
+// us per step with 8 -> 4 elements on rows of 64 and 128 complex points and
+// columns of 128 and 256 points: CH 256^2 10.2 -> 8.3, KPZ 128^2 16.3 -> 12.5,
+// Gray-Scott 256^2 20.2 -> 16.2, model H 256^2 39.7 -> 36.1; 512 EW/KPZ
+// instances of 64^2 .. 512^2 170 -> 174, CH 256^3 156 -> 161.  Rows of 256
+// complex points stay at 8 (with 4: KPZ 512^2 20.3 -> 17.7, but the 512
+// instances 170 -> 183), and so do columns of 512 (with 4, two wavefronts
+// each: 18.3 and 188).  Longer lines take 4 over several wavefronts: 1024-point
+// columns of 16 in one wavefront take CH 1024^2 from 16.4 to 18.7 and model H
+// 1024^2 from 69 to 83.
+//
 // Tile row stride: at least lds_len(nc), since each row's transform works
 // in place, and chosen for the LDS banks (32 of 4 bytes; a store is served
 // 16 lanes at a time, a load 32).  A tile copy moves row pairs: the 16
@@ -37,7 +50,7 @@ __host__ __device__ constexpr int tile_stride(int nc, int lpb)
 
 template <int NC, int LPB, int MAXR = 3>
 struct FRowCfg {
-    static constexpr int E = MAXR > 3 ? (NC >= 4 ? 4 : NC) : (NC >= 1024 ? 16 : (NC >= 512 ? 4 : (NC >= 64 ? 8 : (NC >= 4 ? 4 : NC))));
+    static constexpr int E = MAXR > 3 ? (NC >= 4 ? 4 : NC) : (NC >= 1024 ? 16 : (NC == 256 ? 8 : (NC >= 4 ? 4 : NC)));
     static constexpr int T = NC / E;
     static constexpr int THREADS = LPB * T;
     static constexpr int RS = tile_stride(NC, LPB);
@@ -565,9 +578,7 @@ __device__ __forceinline__ void hermitian_col(float2 (&v)[E], float2 *L, int t, 
 
 template <int N, int TWD>
 struct FColCfg {
-    // 1024- and 2048-point columns: 4 per lane, so that a single large
-    // system still puts several waves on every SIMD
-    static constexpr int E = N >= 4096 ? 16 : (N >= 1024 ? 4 : (N >= 8 ? 8 : N));
+    static constexpr int E = N >= 4096 ? 16 : (N >= 1024 || N == 128 || N == 256 ? 4 : (N >= 8 ? 8 : N));
     static constexpr int T = N / E;
     static constexpr int THREADS = TWD * T;
     static constexpr int LL = lds_len(N);
