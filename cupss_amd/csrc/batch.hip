@@ -294,6 +294,19 @@ static bool lean_op(const FusedInst &a, const TermRefDev &R, LeanOp &O)
     return true;
 }
 
+// D(q) = 1 - dt sum (dynamic) or the sum itself as a polynomial in q^2; false
+// where an operator has 1/|q| or a power above q^6
+static bool implicit_poly(const PresDev *imp, int n, bool dynamic, float dt, float (&d)[4])
+{
+    double s[4] = {dynamic ? 1.0 : 0.0, 0.0, 0.0, 0.0};
+    for (int i = 0; i < n; i++) {
+        if (imp[i].invq != 0 || imp[i].q2n < 0 || imp[i].q2n > 3) return false;
+        s[imp[i].q2n] += dynamic ? -(double)dt * (double)imp[i].c : (double)imp[i].c;
+    }
+    for (int i = 0; i < 4; i++) d[i] = (float)s[i];
+    return true;
+}
+
 // the lean program of a finished 2D descriptor (FusedLean); false where the
 // system is not one
 static bool make_lean(FusedInst &a)
@@ -345,14 +358,78 @@ static bool make_lean(FusedInst &a)
         F.zero = a.zero[f];
     }
     P.nimp = a.u.nimp;
-    double d[4] = {1.0, 0.0, 0.0, 0.0};
-    for (int i = 0; i < a.u.nimp; i++) {
-        const PresDev &D = a.u.imp[i];
-        if (D.invq != 0 || D.q2n < 0 || D.q2n > 3) return false;
-        d[D.q2n] -= (double)a.u.dt * (double)D.c;
+    return implicit_poly(a.u.imp, a.u.nimp, true, a.u.dt, P.d);
+}
+
+// the operators of a descriptor on the general 2D tiles: monomials and
+// polynomials where they are, else table slots (equal ones share a slot), and
+// the tables' memory
+static int make_ops(cupss_system s, FusedInst &a)
+{
+    a.ntab = 0;
+    auto slot = [&a](int kind, int pres0, int npres, int mult_i) {
+        for (int i = 0; i < a.ntab; i++) {
+            const FusedTab &T = a.tab[i];
+            if (T.kind != kind || T.npres != npres || T.mult_i != mult_i || (T.pres0 < 0) != (pres0 < 0)) continue;
+            if (pres0 < 0 || std::memcmp(&a.pool[T.pres0], &a.pool[pres0], sizeof(PresDev) * npres) == 0) return i;
+        }
+        a.tab[a.ntab] = FusedTab{kind, pres0, npres, mult_i};
+        return a.ntab++;
+    };
+    static_assert(FUSED_MAX_GROUPS + FUSED_MAX_TARGETS * (FUSED_MAX_TTERMS + 1) + FUSED_MAX_DERIVED <= FUSED_MAX_TABS,
+                  "a slot for every operator");
+    auto op = [&](FusedOp &O, int pres0, int npres, int mult_i) {
+        const TermRefDev R{nullptr, 0, mult_i, pres0, npres};
+        O.tab = npres == 0 || lean_op(a, R, O.m) ? -1 : slot(TAB_MULT, pres0, npres, mult_i);
+    };
+    auto ref = [&](FusedOp &O, const TermRefDev &R) { op(O, R.pres0, R.npres, R.mult_i); };
+    for (int i = 0; i < a.ngroups; i++) ref(a.gop[i], a.gmul[i]);
+    for (int i = 0; i < a.nder; i++) ref(a.dop[i], a.dmul[i]);
+    for (int i = 0; i < a.nreal; i++) ref(a.lop[i], a.lmul[i]);
+    for (int k = 0; k <= a.ncons; k++) {
+        FusedTarget &TG = a.tgt[k];
+        for (int i = 0; i < TG.nterms; i++) op(TG.term[i].op, TG.term[i].pres0, TG.term[i].npres, TG.term[i].mult_i);
+        if (k > 0 && TG.nimp > 0)
+            TG.div.tab = implicit_poly(a.pool + TG.imp0, TG.nimp, TG.dyn != 0, a.u.dt, TG.div.d)
+                             ? -1
+                             : slot(TG.dyn ? TAB_DYNAMIC : TAB_CONSTRAINT, TG.imp0, TG.nimp, 0);
     }
-    for (int i = 0; i < 4; i++) P.d[i] = (float)d[i];
-    return true;
+    if (a.u.nimp > 0)
+        a.udiv.tab = implicit_poly(a.u.imp, a.u.nimp, true, a.u.dt, a.udiv.d) ? -1 : slot(TAB_DYNAMIC, -1, a.u.nimp, 0);
+    if (s->ftab_n < a.ntab) {
+        // launches in flight may still read the old ones
+        if (s->ftab) HIP_TRY(hipStreamSynchronize(s->stream));
+        (void)hipFree(s->ftab);
+        s->ftab = nullptr;
+        s->ftab_n = 0;
+        if (hipMalloc(&s->ftab, sizeof(float) * (size_t)s->g.nh * a.ntab) != hipSuccess)
+            return fail(CUPSS_ERR_NOMEM, "device allocation failed");
+        s->ftab_n = a.ntab;
+        s->ftab_gen = 0;
+    }
+    a.mtab = s->ftab;
+    return CUPSS_OK;
+}
+
+// an upper bound from the plan: every operator that is not a single monomial
+// without 1/|q|, and the updates with 1/|q|
+size_t fused_table_bytes(cupss_system s)
+{
+    const FusedPlan &P = s->plan;
+    if (!P.ok || s->g.sz > 1) return 0;
+    auto plain = [](const std::vector<cupss_pres> &v) { return v.size() == 1 && v[0].invq == 0; };
+    size_t n = 0;
+    for (auto &grp : P.groups) n += !plain(grp.pres);
+    for (int d : P.derived) n += !plain(s->t[s->f[d].terms[0]].pres);
+    for (size_t k = 0; k <= P.cons.size(); k++) {
+        const FieldRec &F = s->f[k == 0 ? P.phi : P.cons[k - 1]];
+        for (int t : F.terms)
+            if (s->t[t].fac.size() < 2) n += !plain(s->t[t].pres);
+        bool poly = true;
+        for (auto &q : F.imp) poly = poly && q.invq == 0 && q.q2n <= 3;
+        n += !poly;
+    }
+    return sizeof(float) * (size_t)s->g.nh * n;
 }
 
 // device descriptor of system s (its fused plan must be ok); natural: the
@@ -504,6 +581,8 @@ static int describe(cupss_system s, FusedInst &a, bool natural = false)
         }
     }
     if (!natural) a.simple = make_lean(a) ? 1 : 0;
+    if (!natural && !a.simple && !is_elementwise(a))
+        if (int r = make_ops(s, a)) return r;
     if (!natural && !is_elementwise(a)) {
         if (int r = alloc_spec(&s->ft[0], g)) return r;
         if (int r = alloc_spec(&s->ft[1], g)) return r;
@@ -764,6 +843,14 @@ static int refresh(FusedBatch &B)
     }
     if (!B.staged) HIP_TRY(hipEventCreateWithFlags(&B.staged, hipEventDisableTiming));
     HIP_TRY(hipEventRecord(B.staged, B.stream));
+    // operator tables of programs and prefactor values that are new
+    for (size_t i = 0; i < n; i++) {
+        cupss_system s = B.sys[i];
+        if (B.h[i].ntab == 0 || (s->ftab_gen == s->gen && s->ftab_vgen == s->vgen)) continue;
+        HIP_TRY(fused_tables_launch(B.d, (int)i, s->g.nh, B.stream));
+        s->ftab_gen = s->gen;
+        s->ftab_vgen = s->vgen;
+    }
     return CUPSS_OK;
 }
 

@@ -229,6 +229,42 @@ __global__ __launch_bounds__(256) void k_fsettle(const FusedInst *__restrict__ i
         tile_to_nat(s, a, x0, y0, a.dbase[d] < 0 ? a.spec[fin ^ 1] : a.cs[a.dbase[d]][fin ^ 1], a.dout[d], a.dmul[d]);
 }
 
+// ------------------------------------------------------------ operator tables
+
+// every table of one instance, a thread per bin (column-major)
+__global__ __launch_bounds__(256) void k_ftables(const FusedInst *__restrict__ insts, int inst)
+{
+    const FusedInst &a = insts[inst];
+    const long h = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (h >= a.g.nh) return;
+    ColBins<1> cb;
+    col_bins<1, 1>(a.g, (int)(h / a.g.sy), (int)(h % a.g.sy), cb);
+    for (int i = 0; i < a.ntab; i++) {
+        const FusedTab &T = a.tab[i];
+        float m[1];
+        if (T.kind == TAB_MULT) {
+            multiplier_col<1>(a.pool, T.pres0, T.npres, T.mult_i, cb, m);
+        } else {
+            float sum = T.kind == TAB_DYNAMIC ? 1.0f : 0.0f;
+            for (int k = 0; k < T.npres; k++) {
+                const PresDev P = T.pres0 < 0 ? a.u.imp[k] : a.pool[T.pres0 + k];
+                float th = P.c;
+                for (int j = 0; j < P.q2n; j++) th *= cb.q2[0];
+                if (P.invq != 0) {
+                    const float iq = col_iq(cb, 0);
+                    for (int j = 0; j < P.invq; j++) th *= iq;
+                }
+                if (T.kind == TAB_DYNAMIC)
+                    sum -= a.u.dt * th;
+                else
+                    sum += th;
+            }
+            m[0] = T.kind == TAB_CONSTRAINT && cb.zero[0] ? 1.0f : __builtin_amdgcn_rcpf(sum);
+        }
+        gstore(a.mtab, (long)i * a.g.nh + h, m[0]);
+    }
+}
+
 // ------------------------------------------------------------ elementwise
 
 // Instances whose step needs no transform (no products, noise drawn in
@@ -533,6 +569,12 @@ hipError_t fused_small_launch(int nc, int ny, int stored, const FusedInst *inst,
     if (nids <= 0 || k <= 0) return hipSuccess;
     if (nc == 32 && ny == 64) return fsmall_n<32, 64>(stored, inst, ids, nids, n0, k, rel0, s, sets, ts);
     return hipErrorInvalidValue;
+}
+
+hipError_t fused_tables_launch(const FusedInst *inst, int i, long nh, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_ftables, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, s, inst, i);
+    return hipGetLastError();
 }
 
 hipError_t fused_transpose_in_launch(const FusedInst *inst, const FusedBlock *blocks, int nblocks, hipStream_t s)

@@ -54,9 +54,28 @@ enum FusedSrc : int {
     SRC_DYN_NEW = 5,  // stored dynamic field idx after the step (terms of constraint fields)
 };
 
+struct LeanOp {                   // c q^(2 q2n) (i qx)^a (i qy)^b with the sign folded into c
+    float c;
+    int q2n, a, b, mult_i;
+};
+
+// A multiplier as the column pass takes it: the monomial m (tab < 0), or
+// table `tab` of the instance (sums, and operators with 1/|q|)
+struct FusedOp {
+    LeanOp m;
+    int tab;
+};
+// The factor of an update: 1/(d[0] + d[1] q^2 + d[2] q^4 + d[3] q^6) (tab < 0;
+// a constraint's is 1 at q = 0), or table `tab`
+struct FusedDiv {
+    float d[4];
+    int tab;
+};
+
 struct FusedTerm {
     int src, idx;
     int mult_i, pres0, npres;  // multiplier in the pool
+    FusedOp op;
 };
 
 // One field a pass updates: phi (target 0) or stored field c (1 + c)
@@ -66,6 +85,7 @@ struct FusedTarget {
     int g0, g1;      // its product groups [g0, g1)
     int nimp, imp0;  // stored field: implicit prefactors in the pool (constraint: division for q != 0;
                      // dynamic: D(q) = 1 - dt sum)
+    FusedDiv div;    // stored field: its update's factor (nimp > 0)
     int z;           // stored field: index of its real field, -1 if none
     int dyn;         // stored dynamic field: semi-implicit Euler step of its own value
     int fresh;       // stored constraint solved at the start of the pass from the dynamic
@@ -82,15 +102,20 @@ struct FusedTarget {
     float2 *eta;     // NOISE_REAL: R2C_x(xi) rows, column-major (row pass)
 };
 
+// What a table holds: M(q) of the pool prefactors [pres0, pres0 + npres), or
+// 1/(1 - dt sum) or 1/sum (1 at q = 0) over the implicit prefactors there
+// (pres0 < 0: those of phi, u.imp).
+enum FusedTabKind : int { TAB_MULT = 0, TAB_DYNAMIC = 1, TAB_CONSTRAINT = 2 };
+struct FusedTab {
+    int kind, pres0, npres, mult_i;
+};
+constexpr int FUSED_MAX_TABS = 80;    // groups, terms, derived fields, updates
+
 // The program of a simple system in 256 bytes that a workgroup loads at once
 // (lean_tiles.hpp): phi alone (no stored fields; its other terms are
 // constants), at most one product group and two real fields that are phi or
 // monomials of it, a polynomial implicit operator.
 constexpr int LEAN_PRODS = 4;
-struct LeanOp {                   // c q^(2 q2n) (i qx)^a (i qy)^b with the sign folded into c
-    float c;
-    int q2n, a, b, mult_i;
-};
 struct LeanField {
     LeanOp op;
     int lin;                      // 0: the field is phi itself
@@ -164,6 +189,13 @@ struct FusedInst {
     float2 *dout[FUSED_MAX_DERIVED];
     TermRefDev dmul[FUSED_MAX_DERIVED];       // pool
     int dbase[FUSED_MAX_DERIVED];             // u: phi (-1) or stored dynamic field c
+    // The operators of the instances on the general tiles, and ntab column-
+    // major tables of one float per bin, evaluated once (k_ftables)
+    FusedOp gop[FUSED_MAX_GROUPS], lop[FUSED_MAX_REAL], dop[FUSED_MAX_DERIVED];
+    FusedDiv udiv;                            // phi (u.nimp > 0)
+    float *mtab;
+    int ntab;
+    FusedTab tab[FUSED_MAX_TABS];
 };
 
 // Work item of one workgroup: instance and first row / column / tile / bin
@@ -234,6 +266,8 @@ hipError_t fused3d_z_launch(int nz, int twd, const FusedInst *inst, int nc1, int
 // derived fields from phi's spectrum [parity], natural layout
 hipError_t fused3d_derived_launch(const FusedInst *inst, long nh, int parity, hipStream_t s);
 
+// the operator tables of instance i (nh bins)
+hipError_t fused_tables_launch(const FusedInst *inst, int i, long nh, hipStream_t s);
 // natural spectra -> column-major buffer 0 (phi and the stored constraints;
 // blocks: one tile each)
 hipError_t fused_transpose_in_launch(const FusedInst *inst, const FusedBlock *blocks, int nblocks, hipStream_t s);

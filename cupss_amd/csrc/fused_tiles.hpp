@@ -228,20 +228,21 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
         tsl.load(sets);
     }
 
+    // the next field's loads are in flight during a field's transform (model
+    // H 1024^2, five fields: 28.1 -> 27.2 us)
     float2 r[MAXR][E];
+    TileLoad<NC, LPB, RS, TH> tl;
+    if (nreal > 0) tl.issue(a.Z[0], sy, y0, a.kmax[0]);
 #pragma unroll
     for (int f = 0; f < MAXR; f++) {
         if (f < nreal) {
-            // wide rows hold up to FUSED_MAX_REAL fields in registers: one
-            // load in flight there
-            TileLoad<NC, LPB, RS, TH, (MAXR > 3 ? 1 : 4)> tl;
-            tl.issue(a.Z[f], sy, y0, a.kmax[f]);
             if (f == 0 && load_tw) {
                 twl.store(tws, sets);
                 tsl.store(tst, sets);
             }
             tl.commit(tile, a.Z[f], sy, y0, a.kmax[f]);
             __syncthreads();
+            if (f + 1 < MAXR && f + 1 < nreal) tl.issue(a.Z[f + 1], sy, y0, a.kmax[f + 1]);
             float2 xa[E], ya[E], v[E];
 #pragma unroll
             for (int e = 0; e < E; e++) {
@@ -356,6 +357,73 @@ __device__ __forceinline__ void load_col(float2 (&v)[E], const float2 *__restric
     }
 }
 
+// m[e] = table `slot` of the instance at the E bins of a lane's column
+template <int E, int T>
+__device__ __forceinline__ void load_tab(float (&m)[E], const FusedInst &a, int slot, long col, int t, bool active)
+{
+    if (active) {
+        const float *__restrict__ q = a.mtab + (long)slot * a.g.nh + col + t;
+#pragma unroll
+        for (int e = 0; e < E; e++) m[e] = gload(q, (long)e * T);
+    } else {
+#pragma unroll
+        for (int e = 0; e < E; e++) m[e] = 0.f;
+    }
+}
+
+// c q^(2 q2n) qx^a qy^b of the bins of a column, zero where the projection
+// onto real fields drops it (multiplier())
+template <int E>
+__device__ __forceinline__ void mono_col(const LeanOp &O, const ColBins<E> &cb, float (&m)[E])
+{
+    float base = O.c;
+    for (int i = 0; i < O.a; i++) base *= cb.qx;
+    const int parx = O.mult_i + (cb.nyx ? 0 : O.a);
+#pragma unroll
+    for (int e = 0; e < E; e++) m[e] = base;
+    for (int i = 0; i < O.q2n; i++)
+#pragma unroll
+        for (int e = 0; e < E; e++) m[e] *= cb.q2[e];
+    for (int i = 0; i < O.b; i++)
+#pragma unroll
+        for (int e = 0; e < E; e++) m[e] *= cb.qy[e];
+#pragma unroll
+    for (int e = 0; e < E; e++) m[e] = ((parx + (cb.nyy[e] ? 0 : O.b)) & 1) ? 0.0f : m[e];
+}
+
+// The multiplier of a term at the bins of a lane's column.  A monomial stands
+// in the descriptor beside the term and is evaluated; sums of prefactors and
+// operators with 1/|q| are read from the instance's table, with the data they
+// multiply.  A walk over the prefactors is a chain of dependent scalar loads
+// per prefactor (model H 1024^2: 201 scalar loads and 2930 vector
+// instructions per wavefront of the column pass; all from tables 158 and
+// 2040, but 28 bytes a point more traffic, which many instances at once pay
+// for).
+template <int E, int T>
+__device__ __forceinline__ void op_col(const FusedInst &a, const FusedOp &O, const ColBins<E> &cb, long col, int t,
+                                       bool active, float (&m)[E])
+{
+    if (O.tab < 0)
+        mono_col<E>(O.m, cb, m);
+    else
+        load_tab<E, T>(m, a, O.tab, col, t, active);
+}
+// the factor of an update (FusedDiv)
+template <int E, int T>
+__device__ __forceinline__ void div_col(const FusedInst &a, const FusedDiv &D, const ColBins<E> &cb, long col, int t,
+                                        bool active, float (&r)[E])
+{
+    if (D.tab < 0) {
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const float q2 = cb.q2[e];
+            r[e] = __builtin_amdgcn_rcpf(D.d[0] + q2 * (D.d[1] + q2 * (D.d[2] + q2 * D.d[3])));
+        }
+    } else {
+        load_tab<E, T>(r, a, D.tab, col, t, active);
+    }
+}
+
 // Sum of the terms of one target field over the E bins of a lane: product
 // groups (FFT_y of X_g times the group multiplier) and single-field or
 // constant terms.  xv holds X of the first group on entry when `pre`.
@@ -370,16 +438,16 @@ __device__ __forceinline__ void target_sum(const FusedInst &a, const FusedTarget
     for (int e = 0; e < E; e++) acc[e] = make_float2(0.f, 0.f);
     for (int gi = TG.g0; gi < TG.g1; gi++) {
         if (!(pre && gi == TG.g0)) load_col<E, T>(xv, a.X[gi], col, t, active);
-        fft_line<N, E, -1, TW_STAGE, !SKIP, (T <= 64)>(xv, L, t, tws);
         const TermRefDev &GM = a.gmul[gi];
-        multiplier_col<E>(a.pool, GM.pres0, GM.npres, GM.mult_i, cb, m);
+        op_col<E, T>(a, a.gop[gi], cb, col, t, active, m);
+        fft_line<N, E, -1, TW_STAGE, !SKIP, (T <= 64)>(xv, L, t, tws);
 #pragma unroll
         for (int e = 0; e < E; e++) acc[e] = cadd(acc[e], apply_mult(m[e], GM.mult_i, xv[e]));
         line_sync<(T <= 64)>();
     }
     for (int ti = 0; ti < TG.nterms; ti++) {
         const FusedTerm &TR = TG.term[ti];
-        multiplier_col<E>(a.pool, TR.pres0, TR.npres, TR.mult_i, cb, m);
+        op_col<E, T>(a, TR.op, cb, col, t, active, m);
         float2 X[E];
         if (TR.src == SRC_OLD || TR.src == SRC_NEW) {
 #pragma unroll
@@ -390,7 +458,7 @@ __device__ __forceinline__ void target_sum(const FusedInst &a, const FusedTarget
         } else if (TR.src == SRC_DERIVED) {
             const TermRefDev &DM = a.dmul[TR.idx];
             float dm[E];
-            multiplier_col<E>(a.pool, DM.pres0, DM.npres, DM.mult_i, cb, dm);
+            op_col<E, T>(a, a.dop[TR.idx], cb, col, t, active, dm);
             const int b = a.dbase[TR.idx];
             if (b < 0) {
 #pragma unroll
@@ -432,34 +500,6 @@ __device__ __forceinline__ void z_out(const FusedInst &a, int f, const Geom &g, 
     line_sync<(T <= 64)>();
 }
 
-// sum over the pool prefactors [p0, p0 + n) of c q^(2 q2n) |q|^-invq per bin
-// (the implicit operator of a stored field)
-template <int E>
-__device__ __forceinline__ void pool_sum_col(const PresDev *pool, int p0, int n, const ColBins<E> &cb,
-                                             float (&sum)[E])
-{
-#pragma unroll
-    for (int e = 0; e < E; e++) sum[e] = 0.0f;
-    for (int i = 0; i < n; i++) {
-        const PresDev P = pool[p0 + i];
-        float th[E];
-#pragma unroll
-        for (int e = 0; e < E; e++) th[e] = P.c;
-        for (int k = 0; k < P.q2n; k++)
-#pragma unroll
-            for (int e = 0; e < E; e++) th[e] *= cb.q2[e];
-        if (P.invq != 0) {
-#pragma unroll
-            for (int e = 0; e < E; e++) {
-                const float iq = col_iq(cb, e);
-                for (int k = 0; k < P.invq; k++) th[e] *= iq;
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < E; e++) sum[e] += th[e];
-    }
-}
-
 // noise of a stored field over the E bins of a lane, times its amplitude
 // (times 1/sqrt(dt) for a constraint): real-space rows transformed along y,
 // or drawn in spectral space, at the pass's step + step_off
@@ -493,41 +533,22 @@ __device__ __forceinline__ void stored_noise(const FusedInst &a, const FusedTarg
     }
 }
 
-// constraint value: the term sum divided by the implicit operator's sum
-// where q != 0 (setNotDynamic_k, src/field_kernels.cu:130-197)
-template <int E>
-__device__ __forceinline__ void constraint_solve(const FusedInst &a, const FusedTarget &TG, const ColBins<E> &cb,
-                                                 float2 (&v)[E])
+// values of a stored field times its factor: 1/D(q) of a dynamic field, the
+// reciprocal of the implicit operator's sum of a constraint where q != 0
+// (setNotDynamic_k, src/field_kernels.cu:130-197)
+template <int E, int T>
+__device__ __forceinline__ void solve_col(const FusedInst &a, const FusedTarget &TG, const ColBins<E> &cb, long col,
+                                          int t, bool active, float2 (&v)[E])
 {
     if (TG.nimp <= 0) return;
-    float lsum[E];
-    pool_sum_col<E>(a.pool, TG.imp0, TG.nimp, cb, lsum);
+    float r[E];
+    div_col<E, T>(a, TG.div, cb, col, t, active, r);
 #pragma unroll
-    for (int e = 0; e < E; e++)
-        if (!cb.zero[e]) {
-            const float rl = __builtin_amdgcn_rcpf(lsum[e]);
-            v[e].x *= rl;
-            v[e].y *= rl;
-        }
-}
-
-// 1/D(q), D = 1 - dt sum of the pool prefactors [p0, p0 + n) (the implicit
-// operator of a stored dynamic field, summed in implicit_col's order)
-template <int E>
-__device__ __forceinline__ void pool_implicit_col(const PresDev *pool, int p0, int n, float dt, const ColBins<E> &cb,
-                                                  float (&rD)[E])
-{
-    float D[E];
-#pragma unroll
-    for (int e = 0; e < E; e++) D[e] = 1.0f;
-    for (int i = 0; i < n; i++) {
-        float th[E];
-        pool_sum_col<E>(pool, p0 + i, 1, cb, th);
-#pragma unroll
-        for (int e = 0; e < E; e++) D[e] -= dt * th[e];
+    for (int e = 0; e < E; e++) {
+        const float f = !TG.dyn && cb.zero[e] ? 1.0f : r[e];
+        v[e].x *= f;
+        v[e].y *= f;
     }
-#pragma unroll
-    for (int e = 0; e < E; e++) rD[e] = __builtin_amdgcn_rcpf(D[e]);
 }
 
 // Z_f = IFFT_y(mask_f * L_f u) of a real field that is a dynamic field u or
@@ -541,7 +562,7 @@ __device__ __forceinline__ void lz_out(const FusedInst &a, int f, const Geom &g,
     const TermRefDev &LM = a.lmul[f];
     if (LM.npres > 0) {
         float lm[E];
-        multiplier_col<E>(a.pool, LM.pres0, LM.npres, LM.mult_i, cb, lm);
+        op_col<E, T>(a, a.lop[f], cb, col, t, active, lm);
 #pragma unroll
         for (int e = 0; e < E; e++) v[e] = apply_mult(lm[e], LM.mult_i, u[e]);
     } else {
@@ -660,7 +681,7 @@ __device__ __forceinline__ void fcols_tile(const FusedInst &a, int line, int par
                 float2 v[E];
                 target_sum<N, E, T, !CONS>(a, TG, cb, cur, cur, xv, false, parity, active, col, L, t, tws, v);
                 if (TG.noisy) stored_noise<N, E, T, !CONS>(a, TG, cb, kx, step, active, col, L, t, tws, v);
-                constraint_solve<E>(a, TG, cb, v);
+                solve_col<E, T>(a, TG, cb, col, t, active, v);
                 if (edge_wg) hermitian_col<N, E, T>(v, L, t, edge);
                 if (active) {
                     float2 *__restrict__ cout = a.cs[ci][parity];
@@ -687,7 +708,7 @@ __device__ __forceinline__ void fcols_tile(const FusedInst &a, int line, int par
                                     a.key1, eta[e], eta[e + E / 2]);
         }
         float rD[E];
-        if (a.u.nimp > 0) implicit_col<E>(a.u, cb, rD);
+        if (a.u.nimp > 0) div_col<E, T>(a, a.udiv, cb, col, t, active, rD);
 #pragma unroll
         for (int e = 0; e < E; e++) {
             float2 s = cur[e];
@@ -726,24 +747,16 @@ __device__ __forceinline__ void fcols_tile(const FusedInst &a, int line, int par
 #pragma unroll
                 for (int e = 0; e < E; e++) v[e] = make_float2(u0[e].x + dt * v[e].x, u0[e].y + dt * v[e].y);
                 if (TG.noisy) stored_noise<N, E, T, !CONS>(a, TG, cb, kx, step, active, col, L, t, tws, v);
-                if (TG.nimp > 0) {
-                    float rD[E];
-                    pool_implicit_col<E>(a.pool, TG.imp0, TG.nimp, a.u.dt, cb, rD);
-#pragma unroll
-                    for (int e = 0; e < E; e++) {
-                        v[e].x *= rD[e];
-                        v[e].y *= rD[e];
-                    }
-                }
+                solve_col<E, T>(a, TG, cb, col, t, active, v);
             } else if (TG.keep) {
                 // no terms: setNotDynamic_k leaves the value as it is, then
                 // divides it by the implicit operator's sum (if any)
                 const float2 *__restrict__ kin = a.cs[ci][parity];
                 load_col<E, T>(v, kin, col, t, active);
-                constraint_solve<E>(a, TG, cb, v);
+                solve_col<E, T>(a, TG, cb, col, t, active, v);
             } else {
                 if (XDYN && TG.noisy) stored_noise<N, E, T, !CONS>(a, TG, cb, kx, step, active, col, L, t, tws, v);
-                constraint_solve<E>(a, TG, cb, v);
+                solve_col<E, T>(a, TG, cb, col, t, active, v);
             }
             if (edge_wg) hermitian_col<N, E, T>(v, L, t, edge);
             if (active) {

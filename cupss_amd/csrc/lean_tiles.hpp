@@ -168,26 +168,6 @@ __device__ __forceinline__ void lean_rows_tile(const LeanRegs &R, int y0, uint64
     }
 }
 
-// c q^(2 q2n) qx^a qy^b of the bins of a column, zero where the projection
-// onto real fields drops it (multiplier())
-template <int E>
-__device__ __forceinline__ void lean_mult(const LeanOp &O, const ColBins<E> &cb, float (&m)[E])
-{
-    float base = O.c;
-    for (int i = 0; i < O.a; i++) base *= cb.qx;
-    const int parx = O.mult_i + (cb.nyx ? 0 : O.a);
-#pragma unroll
-    for (int e = 0; e < E; e++) m[e] = base;
-    for (int i = 0; i < O.q2n; i++)
-#pragma unroll
-        for (int e = 0; e < E; e++) m[e] *= cb.q2[e];
-    for (int i = 0; i < O.b; i++)
-#pragma unroll
-        for (int e = 0; e < E; e++) m[e] *= cb.qy[e];
-#pragma unroll
-    for (int e = 0; e < E; e++) m[e] = ((parx + (cb.nyy[e] ? 0 : O.b)) & 1) ? 0.0f : m[e];
-}
-
 // Columns line .. line+TWD-1 of one instance (the whole workgroup), as
 // fcols_tile: mode 0 prologue, 1 step from buffer `parity`.
 template <int N, int TWD>
@@ -250,7 +230,7 @@ __device__ __forceinline__ void lean_cols_tile(const LeanRegs &R, int line, int 
             opaque(xv);
             line_sync<WL>();
             float m[E];
-            lean_mult<E>(P.g, cb, m);
+            mono_col<E>(P.g, cb, m);
 #pragma unroll
             for (int e = 0; e < E; e++) {
                 const float2 v = apply_mult(m[e], P.g.mult_i, xv[e]);
@@ -301,7 +281,7 @@ __device__ __forceinline__ void lean_cols_tile(const LeanRegs &R, int line, int 
         float2 v[E];
         if (P.f[f].lin) {
             float m[E];
-            lean_mult<E>(P.f[f].op, cb, m);
+            mono_col<E>(P.f[f].op, cb, m);
 #pragma unroll
             for (int e = 0; e < E; e++) v[e] = apply_mult(m[e], P.f[f].op.mult_i, nw[e]);
         } else {

@@ -127,6 +127,7 @@ extern "C" int cupss_system_destroy(cupss_system s)
         hipFree(c[0]);
         hipFree(c[1]);
     }
+    hipFree(s->ftab);
     hipFree(s->scratch);
     hipFree(s->rtmp);
     hipFree(s->full);
@@ -817,7 +818,7 @@ extern "C" int cupss_system_device_bytes(cupss_system s, size_t *bytes)
     if (s->plan.ok && s->g.sz > 1)  // the 3D fused path's buffers (Z_f, W_f, X_g)
         b += spec * (2 * s->plan.real.size() + s->plan.groups.size());
     else if (s->plan.ok)  // the fused path's buffers, allocated at its first run
-        b += spec * (2 + 2 * s->plan.cons.size() + s->plan.real.size() + s->plan.groups.size());
+        b += spec * (2 + 2 * s->plan.cons.size() + s->plan.real.size() + s->plan.groups.size()) + fused_table_bytes(s);
     b += line_device_bytes(s);
     *bytes = b;
     return CUPSS_OK;

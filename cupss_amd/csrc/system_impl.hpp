@@ -95,6 +95,11 @@ struct cupss_system_t {
     float2 *fx[cupss::FUSED_MAX_GROUPS] = {};
     float2 *ft[2] = {nullptr, nullptr};  // phi's spectrum, column-major, during fused runs
     float2 *fc[cupss::FUSED_MAX_CONS][2] = {};  // stored constraint fields, column-major
+    // operator tables of the general 2D tiles (FusedInst::mtab) and the
+    // program and prefactor values they hold
+    float *ftab = nullptr;
+    int ftab_n = 0;
+    uint64_t ftab_gen = 0, ftab_vgen = 0;
     float2 *fw[cupss::FUSED_MAX_REAL] = {};     // 3D: IFFT_z of the masked real fields (zero off the kept lines)
     // After a fused run, fc[.][cont_buf] holds the stored fields' values of
     // the next step's phase A/B; a run that starts at step cont_step with
@@ -160,6 +165,8 @@ bool line_eligible(cupss_system s);
 int line_steps(cupss_system s, int nsteps);
 void line_release(cupss_system s);
 size_t line_device_bytes(cupss_system s);  // descriptor and tables, made at the first such run
+// bytes of the operator tables a 2D fused system holds (at most)
+size_t fused_table_bytes(cupss_system s);
 int fused_profile(cupss_system s, int on);
 int fused_kernel_time(cupss_system s, float *avg_ms, double *points, char *name, int len);
 }  // namespace cupss

@@ -237,35 +237,7 @@ __device__ __forceinline__ void multiplier_col(const PresDev *__restrict__ pres,
     }
 }
 
-// D(q) = 1 - dt * sum_imp (setDynamic_k) and the noise amplitude, per bin
-template <int E>
-__device__ __forceinline__ void implicit_col(const UpdateArgs &a, const ColBins<E> &cb, float (&rD)[E])
-{
-    float D[E];
-#pragma unroll
-    for (int e = 0; e < E; e++) D[e] = 1.0f;
-    for (int i = 0; i < a.nimp; i++) {
-        const PresDev P = a.imp[i];
-        float th[E];
-#pragma unroll
-        for (int e = 0; e < E; e++) th[e] = P.c;
-        for (int k = 0; k < P.q2n; k++)
-#pragma unroll
-            for (int e = 0; e < E; e++) th[e] *= cb.q2[e];
-        if (P.invq != 0) {
-#pragma unroll
-            for (int e = 0; e < E; e++) {
-                const float iq = col_iq(cb, e);
-                for (int k = 0; k < P.invq; k++) th[e] *= iq;
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < E; e++) D[e] -= a.dt * th[e];
-    }
-#pragma unroll
-    for (int e = 0; e < E; e++) rD[e] = __builtin_amdgcn_rcpf(D[e]);
-}
-
+// the noise amplitude, per bin
 template <int E>
 __device__ __forceinline__ float noise_amplitude_col(const UpdateArgs &a, const ColBins<E> &cb, int e)
 {
