@@ -340,7 +340,11 @@ static void launch_cols(int dir, bool mask, int p, const float2 *in, float2 *out
                            g, p, tw);
 }
 
-// widest valid tile that still gives >= 1024 workgroups, else the narrowest
+// widest valid tile that still gives >= 1024 workgroups, else the narrowest;
+// lines of 1024 points and more stay at 4 (32 adjacent bytes a row): 129
+// workgroups of 4 lines move a 1024^2 half spectrum faster than 513 of one
+// (general program, Cahn-Hilliard, us per step: 1024^2 52 -> 48, 2048^2
+// 112 -> 94), while 512^2 takes 32 with 2 lines and 33 with 4
 template <int N>
 static void cols_n(int dir, bool mask, int p, const float2 *in, float2 *out, long ncols, long stride, long bstride,
                    long nbatch, const Geom &g, hipStream_t s, const float2 *tw)
@@ -350,7 +354,7 @@ static void cols_n(int dir, bool mask, int p, const float2 *in, float2 *out, lon
     for (int w : widths) {
         if (!ColCfg<N>::valid(w)) continue;
         pick = w;
-        if ((ncols + w - 1) / w * nbatch >= 1024) break;
+        if ((ncols + w - 1) / w * nbatch >= 1024 || (N >= 1024 && w == 4)) break;
     }
     switch (pick) {
     case 64:
