@@ -44,7 +44,11 @@ namespace cupss {
 // count each double buffer (phi's spectrum, the stored fields) swaps its
 // halves, so that [0] is again the buffer holding the current state.  The
 // host applies the same changes to its copies (mirror_run_end), so the next
-// run finds the descriptors unchanged and uploads nothing for them.
+// run finds the descriptors unchanged and uploads nothing for them.  Runs
+// that follow each other without an upload, prologue or replay need not even
+// this launch: their kernels take the steps since the last one as offsets of
+// the parity and the counters (FusedBatch::lag).  One-step runs of 256^2
+// diffusion: 6.4 us with a launch per run, 4.0 without.
 __global__ void k_bump_steps(FusedInst *inst, int n, uint32_t by)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -84,6 +88,7 @@ struct Tables {
 
 struct FusedBatch {
     std::vector<cupss_system> sys;
+    uint32_t lag = 0;  // steps taken that the device descriptors do not hold yet (catch_up)
     hipStream_t stream = nullptr;
     bool own_stream = false;
 
@@ -727,6 +732,7 @@ static void default_shapes(FusedBatch::Class &c)
 static int build(FusedBatch &B)
 {
     B.release_tables();
+    B.lag = 0;  // every descriptor is uploaded anew
     B.h.resize(B.sys.size());
     for (size_t i = 0; i < B.sys.size(); i++)
         if (int r = describe(B.sys[i], B.h[i])) return r;
@@ -799,6 +805,18 @@ static int build(FusedBatch &B)
     return CUPSS_OK;
 }
 
+// bring the device descriptors up to the steps taken: before anything but
+// step launches reads them, and before some of them are uploaded anew
+static int catch_up(FusedBatch &B)
+{
+    if (B.lag == 0) return CUPSS_OK;
+    const int ni = (int)B.h.size();
+    hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni, B.lag);
+    B.lag = 0;
+    HIP_TRY(hipGetLastError());
+    return CUPSS_OK;
+}
+
 static bool stale_tables(const FusedBatch &B)
 {
     if (!B.built || B.gens.size() != B.sys.size()) return true;
@@ -827,6 +845,7 @@ static int refresh(FusedBatch &B)
         any = any || B.dirty[i];
     }
     if (!any) return CUPSS_OK;
+    if (int r = catch_up(B)) return r;
     if (B.staged) HIP_TRY(hipEventSynchronize(B.staged));
     for (size_t i = 0; i < n;) {
         if (!B.dirty[i]) {
@@ -862,6 +881,8 @@ static int launch_prologue(FusedBatch &B)
     bool all = true;
     for (size_t i = 0; i < B.h.size(); i++)
         if (!B.is_elem[i] && !B.h[i].resume) all = false;
+    if (!all)
+        if (int r = catch_up(B)) return r;
     if (B.ntb > 0 && !all) HIP_TRY(fused_transpose_in_launch(B.d, B.tb, B.ntb, B.stream));
     for (auto &c : B.classes) {
         bool resumed = true;
@@ -1178,8 +1199,10 @@ static int flush(FusedBatch &B)
 {
     if (!B.settle_pending) return CUPSS_OK;
     B.settle_pending = false;
-    // the run's last k_bump_steps left the final state in buffer [0] and
-    // the last step's start in [1]
+    // with the counters caught up, the final state is in buffer [0] and the
+    // last step's start in [1]
+    if (B.ntb > 0)
+        if (int r = catch_up(B)) return r;
     if (B.ntb > 0) HIP_TRY(fused_settle_launch(B.d, B.tb, B.ntb, 0, B.stream));
     bool waits = false;
     for (cupss_system s : B.sys) {
@@ -1273,6 +1296,7 @@ static int run(FusedBatch &B, int nsteps)
             B.gpcount = B.pcount;
             B.gpsteps = B.psteps;
         }
+        if (int r = catch_up(B)) return r;
         while (nsteps - done >= K) {
             HIP_TRY(hipGraphLaunch(B.gexec, B.stream));
             done += K;
@@ -1285,13 +1309,14 @@ static int run(FusedBatch &B, int nsteps)
         mirror_run_end(B.h, (uint32_t)done);
     }
     if (nsteps > done) {
-        if (int r = launch_all(B, done, nsteps - done, done)) return r;
-        // the device's step counters and buffer order follow the steps, so
-        // that the next run's descriptors need no upload for them
-        const int ni = (int)B.h.size();
-        hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni,
-                           (uint32_t)(nsteps - done));
-        HIP_TRY(hipGetLastError());
+        // offsets from the descriptors as the device holds them
+        if ((uint64_t)B.lag + (uint64_t)(nsteps - done) > (1u << 30))
+            if (int r = catch_up(B)) return r;
+        const int lag = (int)B.lag;
+        if (int r = launch_all(B, lag, nsteps - done, 0)) return r;
+        // the next run's descriptors need no upload for the counters and the
+        // buffer order: they follow the steps
+        B.lag += (uint32_t)(nsteps - done);
         mirror_run_end(B.h, (uint32_t)(nsteps - done));
     }
     B.steps_run += nsteps;
