@@ -111,6 +111,8 @@ struct FusedBatch {
     std::vector<char> is_elem;  // per instance
     FusedBlock *eb = nullptr;   // elementwise: FUSED_ELEM_BLOCK pairs of bins per block
     int neb = 0;
+    FusedBlock *leb = nullptr;  // the same for the simple ones
+    int nleb = 0;
     FusedBlock *tb = nullptr;   // transpose tiles of the transform instances
     int ntb = 0;
     hipEvent_t done = nullptr;  // recorded after each run; member streams wait on it
@@ -194,6 +196,9 @@ struct FusedBatch {
         hipFree(eb);
         eb = nullptr;
         neb = 0;
+        hipFree(leb);
+        leb = nullptr;
+        nleb = 0;
         hipFree(tb);
         tb = nullptr;
         ntb = 0;
@@ -750,13 +755,14 @@ static int build(FusedBatch &B)
     }
     std::map<std::pair<int, int>, int> cls;
     B.is_elem.assign(B.h.size(), 0);
-    std::vector<FusedBlock> tiles, er;
+    std::vector<FusedBlock> tiles, er, ler;
     for (size_t i = 0; i < B.h.size(); i++) {
         const FusedInst &a = B.h[i];
         if (is_elementwise(a)) {
             B.elem.push_back((int)i);
             B.is_elem[i] = 1;
-            for (long h0 = 0; h0 < a.g.nh / 2; h0 += FUSED_ELEM_BLOCK) er.push_back(FusedBlock{(int)i, (int)h0});
+            for (long h0 = 0; h0 < a.g.nh / 2; h0 += FUSED_ELEM_BLOCK)
+                (a.simple ? ler : er).push_back(FusedBlock{(int)i, (int)h0});
             continue;
         }
         int stored = a.ncons > 0 ? 1 : 0;
@@ -791,6 +797,7 @@ static int build(FusedBatch &B)
         }
     }
     if (int r = upload_blocks(er, &B.eb, &B.neb)) return r;
+    if (int r = upload_blocks(ler, &B.leb, &B.nleb)) return r;
     if (int r = upload_blocks(tiles, &B.tb, &B.ntb)) return r;
     if (B.profile)
         if (int r = retable(B)) return r;
@@ -951,7 +958,7 @@ static int launch_all(FusedBatch &B, int n0, int k, int rel0)
         for (int i : B.classes[ci].insts) cost += (double)B.h[i].g.n * (4 + B.h[i].nreal + B.h[i].ngroups);
         items.push_back({cost, (int)ci});
     }
-    if (B.neb > 0) {
+    if (B.neb + B.nleb > 0) {
         double cost = 0;
         for (int i : B.elem) cost += (double)B.h[i].g.n;
         items.push_back({cost, -1});
@@ -992,7 +999,8 @@ static int launch_all(FusedBatch &B, int n0, int k, int rel0)
         if (items[it].second >= 0) {
             if (int r = launch_class(B, (size_t)items[it].second, n0, k, rel0, st)) return r;
         } else {
-            HIP_TRY(fused_elem_launch(B.d, B.eb, B.neb, n0 & 1, (uint32_t)(n0 - rel0), k, st));
+            if (B.neb > 0) HIP_TRY(fused_elem_launch(B.d, B.eb, B.neb, n0 & 1, (uint32_t)(n0 - rel0), k, st));
+            if (B.nleb > 0) HIP_TRY(lean_elem_launch(B.d, B.leb, B.nleb, n0 & 1, (uint32_t)(n0 - rel0), k, st));
         }
     }
     for (int j = 1; j < L; j++) {

@@ -280,5 +280,8 @@ hipError_t fused_settle_launch(const FusedInst *inst, const FusedBlock *blocks, 
 // from the last step's start
 hipError_t fused_elem_launch(const FusedInst *inst, const FusedBlock *blocks, int nblocks, int parity,
                              uint32_t step_rel, int nsteps, hipStream_t s);
+// the same where every instance is simple
+hipError_t lean_elem_launch(const FusedInst *inst, const FusedBlock *blocks, int nblocks, int parity,
+                            uint32_t step_rel, int nsteps, hipStream_t s);
 
 }  // namespace cupss
