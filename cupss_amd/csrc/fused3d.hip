@@ -28,12 +28,27 @@ namespace cupss {
 // others stay zero from allocation.  The systems have no stored constraint
 // fields (the host checks).
 
+// Rows of 128 complex points take 8 elements a lane, not the 4 of the 2D tile
+// (FRowCfg): a large box fills the chip with rows, so the fewer exchanges win
+// (CH 256^3: 163.5 us per step with 4, 158.8 with 8).
 template <int NC, int LPB, int MAXR>
-__global__ __launch_bounds__((FRowCfg<NC, LPB, MAXR>::THREADS)) void k_f3rows(const FusedInst *__restrict__ insts,
+struct F3RowCfg {
+    static constexpr int E = NC == 128 && MAXR <= 3 ? 8 : FRowCfg<NC, LPB, MAXR>::E;
+    static constexpr int T = NC / E;
+    static constexpr int THREADS = LPB * T;
+    static constexpr int RS = tile_stride(NC, LPB);
+    static constexpr bool valid()
+    {
+        return THREADS >= 16 && THREADS <= 512 && (LPB * RS + 2 * NC + tw_stage_alloc(NC, E)) * 8 <= 150 * 1024;
+    }
+};
+
+template <int NC, int LPB, int MAXR>
+__global__ __launch_bounds__((F3RowCfg<NC, LPB, MAXR>::THREADS)) void k_f3rows(const FusedInst *__restrict__ insts,
                                                                            uint32_t step_rel,
                                                                            const float2 *__restrict__ sets)
 {
-    using C = FRowCfg<NC, LPB, MAXR>;
+    using C = F3RowCfg<NC, LPB, MAXR>;
     constexpr int E = C::E, T = C::T, RS = C::RS;
     __shared__ float2 tws[2 * NC];
     __shared__ __align__(16) float2 tst[tw_stage_alloc(NC, E)];
@@ -453,11 +468,11 @@ __global__ __launch_bounds__(256) void k_f3der(const FusedInst *__restrict__ ins
 template <int NC, int MAXR>
 static hipError_t f3rows_n(const FusedInst *inst, long nrows, uint32_t step_rel, hipStream_t s, const float2 *sets)
 {
-    constexpr int T = FRowCfg<NC, 1, MAXR>::T;
+    constexpr int T = F3RowCfg<NC, 1, MAXR>::T;
     constexpr int LPB = T >= 256 ? 1 : 256 / T;  // 256 threads a workgroup
-    static_assert(FRowCfg<NC, LPB, MAXR>::valid(), "3D row tile");
+    static_assert(F3RowCfg<NC, LPB, MAXR>::valid(), "3D row tile");
     hipLaunchKernelGGL((k_f3rows<NC, LPB, MAXR>), dim3((unsigned)((nrows + LPB - 1) / LPB)),
-                       dim3(FRowCfg<NC, LPB, MAXR>::THREADS), 0, s, inst, step_rel, sets);
+                       dim3(F3RowCfg<NC, LPB, MAXR>::THREADS), 0, s, inst, step_rel, sets);
     return hipGetLastError();
 }
 
