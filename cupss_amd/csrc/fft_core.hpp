@@ -448,4 +448,70 @@ __device__ __forceinline__ void fft_line(float2 (&v)[E], float2 *lds, int t, con
     }
 }
 
+// Two lines at a time, the second ls entries behind the first: the
+// arithmetic of Stockham on each, one synchronisation and one set of twiddle
+// reads for both.  A line over several wavefronts waits at a barrier in every
+// exchange; with two lines it does so half as often per line, and the second
+// line's butterflies fill the latency of the first's LDS accesses.
+template <int N, int E, int DIR, int NS, bool OUT_LDS, bool WL>
+struct StockhamPair {
+    using S = Stockham<N, E, DIR, NS, TW_STAGE, OUT_LDS, WL>;
+    static constexpr int T = S::T, R = S::R;
+    static constexpr bool LAST = S::LAST;
+    __device__ __forceinline__ static void run(float2 (&v)[2][E], float2 *lds, int ls, int t,
+                                               const float2 *__restrict__ tw)
+    {
+        if constexpr (NS < N) {
+#pragma unroll
+            for (int b = 0; b < E / R; b++) {
+                const int j = t + b * T;
+                const int k = j & (NS - 1);
+                float2 w[R];
+                if constexpr (NS > 1) {
+                    const float2 *__restrict__ st = tw + tw_stage_base(N, E, NS) + k;
+#pragma unroll
+                    for (int r = 1; r < R; r++) w[r] = tw_dir<DIR>(st[(r - 1) * NS]);
+                }
+#pragma unroll
+                for (int m = 0; m < 2; m++) {
+                    float2 a[R];
+#pragma unroll
+                    for (int r = 0; r < R; r++) a[r] = v[m][b + r * (E / R)];
+                    if constexpr (NS > 1) {
+#pragma unroll
+                        for (int r = 1; r < R; r++) a[r] = cmul(a[r], w[r]);
+                    }
+                    Dft<R, DIR>::run(a);
+                    if constexpr (LAST && !OUT_LDS) {
+#pragma unroll
+                        for (int r = 0; r < R; r++) v[m][b + r * (E / R)] = a[r];
+                    } else {
+                        const int wb = m * ls + S::pad((j - k) * R + k);
+#pragma unroll
+                        for (int r = 0; r < R; r++) lds[wb + S::pad(r * NS)] = a[r];
+                    }
+                }
+            }
+            if constexpr (!(LAST && !OUT_LDS)) {
+                line_sync<WL>();
+#pragma unroll
+                for (int m = 0; m < 2; m++) {
+                    const int rb = m * ls + S::pad(t);
+#pragma unroll
+                    for (int e = 0; e < E; e++) v[m][e] = lds[rb + S::pad(e * T)];
+                }
+                if constexpr (!LAST) line_sync<WL>();
+            }
+            StockhamPair<N, E, DIR, NS * R, OUT_LDS, WL>::run(v, lds, ls, t, tw);
+        }
+    }
+};
+
+// fft_line of two lines (N > 1, stage twiddles)
+template <int N, int E, int DIR, bool OUT_LDS = true, bool WL = false>
+__device__ __forceinline__ void fft_pair(float2 (&v)[2][E], float2 *lds, int ls, int t, const float2 *__restrict__ tw)
+{
+    StockhamPair<N, E, DIR, 1, OUT_LDS, WL>::run(v, lds, ls, t, tw);
+}
+
 }  // namespace cupss

@@ -55,7 +55,7 @@ __global__ __launch_bounds__((FRowCfg<NC, LPB, MAXR>::THREADS)) void k_frows(con
     using C = FRowCfg<NC, LPB, MAXR>;
     __shared__ __align__(16) float2 tws[2 * NC];
     __shared__ __align__(16) float2 tst[tw_stage_alloc(NC, C::E)];
-    __shared__ float2 tile[LPB * C::RS];
+    __shared__ float2 tile[C::LEN];
     const FusedBlock blk = blocks[blockIdx.x];
     if (blk.inst < 0) return;
     frows_tile<NC, LPB, MAXR>(insts[blk.inst], blk.line, step_rel, sets, true, tws, tst, tile);
@@ -98,8 +98,8 @@ struct FSmallCfg {
     static constexpr int THREADS = 512;
     static constexpr int LPB = THREADS / FRowCfg<NC, 1, 3>::T;
     static constexpr int TWD = THREADS / FColCfg<N, 1>::T;
-    static constexpr int LDSN = LPB * FRowCfg<NC, LPB, 3>::RS > TWD * FColCfg<N, TWD>::LL
-                                    ? LPB * FRowCfg<NC, LPB, 3>::RS
+    static constexpr int LDSN = FRowCfg<NC, LPB, 3>::LEN > TWD * FColCfg<N, TWD>::LL
+                                    ? FRowCfg<NC, LPB, 3>::LEN
                                     : TWD * FColCfg<N, TWD>::LL;
     static constexpr bool valid()
     {

@@ -54,9 +54,18 @@ struct FRowCfg {
     static constexpr int T = NC / E;
     static constexpr int THREADS = LPB * T;
     static constexpr int RS = tile_stride(NC, LPB);
+    // Two fields, and two products, at a time through their transforms: half
+    // the barriers of a line over several wavefronts and one line's LDS
+    // latency under the other's butterflies.  us per step, Gray-Scott 64^2
+    // 16.3 -> 15.9, 128^2 16.3 -> 15.1, 256^2 16.7 -> 16.0, 1024x512 26.3 ->
+    // 25.1.  Not the wide kernel, whose LDS and registers are the limit of a
+    // batch: model H 1024^2 alone 64.7 -> 63.8, but a mixed batch 122 -> 128.
+    // Not 16 elements a lane (registers).
+    static constexpr bool PAIR = MAXR > 1 && MAXR <= 3 && E <= 8;
+    static constexpr int LEN = (PAIR ? 2 : 1) * LPB * RS;
     static constexpr bool valid()
     {
-        return THREADS >= 16 && THREADS <= 512 && (LPB * RS + 2 * NC + tw_stage_alloc(NC, E)) * 8 <= 150 * 1024;
+        return THREADS >= 16 && THREADS <= 512 && (LEN + 2 * NC + tw_stage_alloc(NC, E)) * 8 <= 150 * 1024;
     }
 };
 
@@ -203,6 +212,38 @@ __device__ __forceinline__ void r2c_tile(float2 (&v)[E], float2 *L, int t, const
     __syncthreads();
 }
 
+// r2c_tile of two rows, the second's LDS ls entries behind the first's
+template <int NC, int E, int T>
+__device__ __forceinline__ void r2c_pair(float2 (&v)[2][E], float2 *L, int ls, int t, const float2 *tws,
+                                         const float2 *ftw)
+{
+    fft_pair<NC, E, -1, true, (T <= 64)>(v, L, ls, t, ftw);
+    float2 o[2][E], z0[2];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int k = t + e * T;
+        const float2 tw = tw_lookup<-1, 2 * NC>(tws, k, 2 * NC);
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            const float2 A = v[m][e];
+            const float2 B = cconj(L[m * ls + lpad((NC - k) & (NC - 1))]);
+            const float2 xe = cscale(cadd(A, B), 0.5f);
+            const float2 xo = cscale(mul_i<-1>(csub(A, B)), 0.5f);
+            o[m][e] = k == 0 ? make_float2(xe.x + xo.x, 0.0f) : cadd(xe, cmul(tw, xo));
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < 2; m++) z0[m] = L[m * ls + lpad(0)];
+    line_sync<(T <= 64)>();  // every read of the transforms' LDS lines is done
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+#pragma unroll
+        for (int e = 0; e < E; e++) L[m * ls + t + e * T] = o[m][e];
+        if (t == 0) L[m * ls + NC] = make_float2(z0[m].x - z0[m].y, 0.0f);
+    }
+    __syncthreads();
+}
+
 // Rows y0 .. y0+LPB-1 of one instance (the whole workgroup).  load_tw:
 // copy the twiddle tables into tws (2NC points) and tst (the NC-point
 // transform's stage tables) first (otherwise they are there already).
@@ -228,35 +269,61 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
         tsl.load(sets);
     }
 
-    // the next field's loads are in flight during a field's transform (model
-    // H 1024^2, five fields: 28.1 -> 27.2 us)
+    // Fields one by one or in pairs (FRowCfg::PAIR).  The next fields' loads
+    // are in flight during a transform (model H 1024^2, five fields: 28.1 ->
+    // 27.2 us).
+    constexpr int P = C::PAIR ? 2 : 1, TS = LPB * RS;
     float2 r[MAXR][E];
-    TileLoad<NC, LPB, RS, TH> tl;
-    if (nreal > 0) tl.issue(a.Z[0], sy, y0, a.kmax[0]);
+    TileLoad<NC, LPB, RS, TH> tl[P];
 #pragma unroll
-    for (int f = 0; f < MAXR; f++) {
+    for (int m = 0; m < P; m++)
+        if (m < nreal) tl[m].issue(a.Z[m], sy, y0, a.kmax[m]);
+#pragma unroll
+    for (int f = 0; f < MAXR; f += P) {
         if (f < nreal) {
+            const bool two = P == 2 && f + 1 < MAXR && f + 1 < nreal;
             if (f == 0 && load_tw) {
                 twl.store(tws, sets);
                 tsl.store(tst, sets);
             }
-            tl.commit(tile, a.Z[f], sy, y0, a.kmax[f]);
+            tl[0].commit(tile, a.Z[f], sy, y0, a.kmax[f]);
+            if constexpr (P == 2)
+                if (two) tl[1].commit(tile + TS, a.Z[f + 1], sy, y0, a.kmax[f + 1]);
             __syncthreads();
-            if (f + 1 < MAXR && f + 1 < nreal) tl.issue(a.Z[f + 1], sy, y0, a.kmax[f + 1]);
-            float2 xa[E], ya[E], v[E];
 #pragma unroll
-            for (int e = 0; e < E; e++) {
-                const int k = t + e * T;
-                xa[e] = L[k];
-                ya[e] = L[NC - k];
+            for (int m = 0; m < P; m++)
+                if (f + P + m < MAXR && f + P + m < nreal) tl[m].issue(a.Z[f + P + m], sy, y0, a.kmax[f + P + m]);
+            float2 v[P][E];
+#pragma unroll
+            for (int m = 0; m < P; m++) {
+                if (m == 0 || two) {
+                    float2 xa[E], ya[E];
+#pragma unroll
+                    for (int e = 0; e < E; e++) {
+                        const int k = t + e * T;
+                        xa[e] = L[m * TS + k];
+                        ya[e] = L[m * TS + NC - k];
+                    }
+                    c2r_prep<NC, E, T>(xa, ya, t, v[m], tws);
+                }
             }
             // the row's part of the tile becomes its transform's LDS (the
             // row's lanes are the only ones that read or write it from here)
             line_sync<(T <= 64)>();
-            c2r_prep<NC, E, T>(xa, ya, t, v, tws);
-            fft_line<NC, E, +1, TW_STAGE, false, (T <= 64)>(v, L, t, tst);
+            if constexpr (P == 2) {
+                if (two)
+                    fft_pair<NC, E, +1, false, (T <= 64)>(v, L, TS, t, tst);
+                else
+                    fft_line<NC, E, +1, TW_STAGE, false, (T <= 64)>(v[0], L, t, tst);
+            } else {
+                fft_line<NC, E, +1, TW_STAGE, false, (T <= 64)>(v[0], L, t, tst);
+            }
 #pragma unroll
-            for (int e = 0; e < E; e++) r[f][e] = cscale(v[e], a.scale);
+            for (int m = 0; m < P; m++)
+                if (f + m < MAXR && (m == 0 || two)) {
+#pragma unroll
+                    for (int e = 0; e < E; e++) r[f + m < MAXR ? f + m : 0][e] = cscale(v[m][e], a.scale);
+                }
             __syncthreads();
         }
     }
@@ -267,8 +334,9 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
         }
         __syncthreads();  // twiddles
     }
-    for (int gi = 0; gi < a.ngroups; gi++) {
-        float2 v[E];
+    // v = group gi's products: coef * prod_f r_f^cnt_f (static field index,
+    // uniform powers: no dynamic indexing, so r stays in registers)
+    auto products = [&](int gi, float2(&v)[E]) {
 #pragma unroll
         for (int e = 0; e < E; e++) v[e] = make_float2(0.f, 0.f);
         for (int pi = a.pg0[gi]; pi < a.pg0[gi + 1]; pi++) {
@@ -276,8 +344,6 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
             const float c0 = a.coef[pi];
 #pragma unroll
             for (int e = 0; e < E; e++) p[e] = make_float2(c0, c0);
-            // product = coef * prod_f r_f^cnt_f: static field index, uniform
-            // powers (no dynamic indexing, so r stays in registers)
 #pragma unroll
             for (int f = 0; f < MAXR; f++)
                 for (int c = 0; c < a.cnt[pi][f]; c++) {
@@ -290,6 +356,21 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
 #pragma unroll
             for (int e = 0; e < E; e++) v[e] = cadd(v[e], p[e]);
         }
+    };
+    int gi = 0;
+    if constexpr (P == 2)
+        for (; gi + 1 < a.ngroups; gi += 2) {
+            float2 v[2][E];
+            products(gi, v[0]);
+            products(gi + 1, v[1]);
+            r2c_pair<NC, E, T>(v, L, TS, t, tws, tst);
+            tile_store<NC, LPB, RS, TH>(a.X[gi], tile, sy, y0);
+            tile_store<NC, LPB, RS, TH>(a.X[gi + 1], tile + TS, sy, y0);
+            __syncthreads();
+        }
+    for (; gi < a.ngroups; gi++) {
+        float2 v[E];
+        products(gi, v);
         r2c_tile<NC, E, T, TW_STAGE>(v, L, t, tws, tst);
         tile_store<NC, LPB, RS, TH>(a.X[gi], tile, sy, y0);
         __syncthreads();
