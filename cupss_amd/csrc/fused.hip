@@ -537,7 +537,8 @@ hipError_t fused_cols_launch(int ny, int twd, int stored, const FusedInst *inst,
 // per pass; on 128^2 one CU's vector issue is the bound and two launches per
 // step over the chip are faster.  us per step, one workgroup / two launches:
 // CH 64^2 5.9 / 8.2, KPZ 64^2 11.8 / 12.9, Gray-Scott 64^2 16.6 / 18.0; KPZ
-// 128^2 42 / 16, Gray-Scott 128^2 48 / 21.  Many instances at once hide either
+// 128^2 42 / 16, Gray-Scott 128^2 48 / 21 (two launches now take 12.5 and 15.1,
+// see FRowCfg and FColCfg).  Many instances at once hide either
 // (512 EW/KPZ instances: 169 us per step with 128^2 on one workgroup each or
 // not).
 bool fused_small_class(int nc, int ny, int width) { return width <= 3 && nc == 32 && ny == 64; }

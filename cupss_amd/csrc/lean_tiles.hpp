@@ -12,7 +12,8 @@
 // implicit operator is one polynomial in q^2.  Measured, us per step, general
 // tiles -> these: CH 256^2 11.9 -> 10.1, CH 1024^2 17.6 -> 16.3, KPZ 512^2
 // with real-space noise 22.4 -> 20.1; 512 EW/KPZ instances of 64^2 .. 512^2
-// 183 -> 169.  What bounds them now: one or two wavefronts a SIMD and two
+// 183 -> 169 (with the elements a lane of FRowCfg and FColCfg, CH 256^2 takes
+// 8.2 today).  What bounds them now: one or two wavefronts a SIMD and two
 // launches a step on a small grid, vector issue on many instances.
 #pragma once
 #include <hip/hip_runtime.h>
