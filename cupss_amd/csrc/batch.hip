@@ -49,11 +49,18 @@ namespace cupss {
 // this launch: their kernels take the steps since the last one as offsets of
 // the parity and the counters (FusedBatch::lag).  One-step runs of 256^2
 // diffusion: 6.4 us with a launch per run, 4.0 without.
-__global__ void k_bump_steps(FusedInst *inst, int n, uint32_t by)
+//
+// once != 0: a launch inside a caller's graph that must take effect at the
+// graph's first replay only.
+__global__ void k_bump_steps(FusedInst *inst, int n, uint32_t by, uint32_t once)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     FusedInst &a = inst[i];
+    if (once != 0) {
+        if (a.caught >= once) return;
+        a.caught = once;
+    }
     a.step_base += by;
     if (by & 1) {
         float2 *t = a.spec[0];
@@ -89,6 +96,11 @@ struct Tables {
 struct FusedBatch {
     std::vector<cupss_system> sys;
     uint32_t lag = 0;  // steps taken that the device descriptors do not hold yet (catch_up)
+    // A caller recorded runs into a graph of its own, which it may replay at
+    // any time: the offsets in those launches count from descriptors that
+    // hold every step, so no run lets them lag any more.
+    bool recorded = false;
+    uint32_t once = 0;  // the last catch-up inside a caller's graph (FusedInst::caught)
     hipStream_t stream = nullptr;
     bool own_stream = false;
 
@@ -738,9 +750,11 @@ static int build(FusedBatch &B)
 {
     B.release_tables();
     B.lag = 0;  // every descriptor is uploaded anew
+    B.recorded = false;  // a caller's graph of runs on the released tables cannot be replayed
     B.h.resize(B.sys.size());
     for (size_t i = 0; i < B.sys.size(); i++)
         if (int r = describe(B.sys[i], B.h[i])) return r;
+    for (FusedInst &a : B.h) a.caught = B.once;
     if (B.dcap < B.h.size()) {
         HIP_TRY(hipStreamSynchronize(B.stream));
         hipFree(B.d);
@@ -812,13 +826,23 @@ static int build(FusedBatch &B)
     return CUPSS_OK;
 }
 
+// whether the launches of this batch are being recorded into a caller's graph
+static bool recording(const FusedBatch &B)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(B.stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 // bring the device descriptors up to the steps taken: before anything but
 // step launches reads them, and before some of them are uploaded anew
 static int catch_up(FusedBatch &B)
 {
     if (B.lag == 0) return CUPSS_OK;
     const int ni = (int)B.h.size();
-    hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni, B.lag);
+    const uint32_t once = recording(B) ? ++B.once : 0;
+    if (once != 0)
+        for (FusedInst &a : B.h) a.caught = once;
+    hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni, B.lag, once);
     B.lag = 0;
     HIP_TRY(hipGetLastError());
     return CUPSS_OK;
@@ -845,6 +869,7 @@ static int refresh(FusedBatch &B)
     for (size_t i = 0; i < n; i++) {
         if (B.vgens[i] != B.sys[i]->vgen) {  // new prefactor values, same structure: new pool
             if (int r = describe(B.sys[i], B.h[i])) return r;
+            B.h[i].caught = B.once;
             B.vgens[i] = B.sys[i]->vgen;
             B.dirty[i] = 1;
         }
@@ -1291,7 +1316,7 @@ static int run(FusedBatch &B, int nsteps)
             if (rc == CUPSS_OK) {
                 const int ni = (int)B.h.size();
                 hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni,
-                                   (uint32_t)K);
+                                   (uint32_t)K, 0u);
             }
             hipGraph_t g = nullptr;
             HIP_TRY(hipStreamEndCapture(B.stream, &g));
@@ -1317,14 +1342,21 @@ static int run(FusedBatch &B, int nsteps)
         mirror_run_end(B.h, (uint32_t)done);
     }
     if (nsteps > done) {
+        B.recorded = B.recorded || recording(B);
         // offsets from the descriptors as the device holds them
-        if ((uint64_t)B.lag + (uint64_t)(nsteps - done) > (1u << 30))
+        if (B.recorded || (uint64_t)B.lag + (uint64_t)(nsteps - done) > (1u << 30))
             if (int r = catch_up(B)) return r;
         const int lag = (int)B.lag;
         if (int r = launch_all(B, lag, nsteps - done, 0)) return r;
         // the next run's descriptors need no upload for the counters and the
         // buffer order: they follow the steps
         B.lag += (uint32_t)(nsteps - done);
+        if (B.recorded) {
+            const int ni = (int)B.h.size();
+            hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni, B.lag, 0u);
+            HIP_TRY(hipGetLastError());
+            B.lag = 0;
+        }
         mirror_run_end(B.h, (uint32_t)(nsteps - done));
     }
     B.steps_run += nsteps;

@@ -149,6 +149,7 @@ struct alignas(64) FusedLean {
 struct FusedInst {
     FusedLean lean;
     int simple;                               // lean holds the system
+    uint32_t caught;                          // the last one-time catch-up taken (k_bump_steps)
     Geom g;
     float2 *spec[2];                          // phi's spectrum: [parity] in, [parity^1] out
     float2 *nat;                              // the system's spectrum (natural layout), transform instances
