@@ -826,20 +826,13 @@ static int build(FusedBatch &B)
     return CUPSS_OK;
 }
 
-// whether the launches of this batch are being recorded into a caller's graph
-static bool recording(const FusedBatch &B)
-{
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(B.stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
-}
-
 // bring the device descriptors up to the steps taken: before anything but
 // step launches reads them, and before some of them are uploaded anew
 static int catch_up(FusedBatch &B)
 {
     if (B.lag == 0) return CUPSS_OK;
     const int ni = (int)B.h.size();
-    const uint32_t once = recording(B) ? ++B.once : 0;
+    const uint32_t once = recording(B.stream) ? ++B.once : 0;
     if (once != 0)
         for (FusedInst &a : B.h) a.caught = once;
     hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni, B.lag, once);
@@ -1342,7 +1335,7 @@ static int run(FusedBatch &B, int nsteps)
         mirror_run_end(B.h, (uint32_t)done);
     }
     if (nsteps > done) {
-        B.recorded = B.recorded || recording(B);
+        B.recorded = B.recorded || recording(B.stream);
         // offsets from the descriptors as the device holds them
         if (B.recorded || (uint64_t)B.lag + (uint64_t)(nsteps - done) > (1u << 30))
             if (int r = catch_up(B)) return r;

@@ -545,8 +545,7 @@ bool line_eligible(cupss_system s)
             // the upload cannot be recorded into a graph: a caller's capture
             // that starts before the program was uploaded records the general
             // program's launches
-            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-            if (hipStreamIsCapturing(s->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) return false;
+            if (recording(s->stream)) return false;
         }
     }
     return S->ok;

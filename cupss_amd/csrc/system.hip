@@ -39,6 +39,12 @@ int cupss::fail(int code, const std::string &msg)
     return code;
 }
 
+bool cupss::recording(hipStream_t stream)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 static bool is_pow2(int v) { return v >= 1 && (v & (v - 1)) == 0; }
 
 extern "C" const char *cupss_last_error(void) { return g_last_error.c_str(); }
@@ -780,7 +786,13 @@ extern "C" int cupss_system_advance(cupss_system s, int nsteps)
     if (int r = check_sys(s)) return r;
     if (!s->prepared) return fail(CUPSS_ERR_STATE, "cupss_system_prepare must be called before advancing");
     if (nsteps <= 0) return CUPSS_OK;
-    if (s->path_mode == 0 && s->plan.ok && !hooks_present(s) && fused_noise_ok(s)) {
+    // Real-space noise in 3D: a caller's graph records the general program's
+    // launches, which need no set-up (the fused step's first run uploads its
+    // descriptor and allocates, and a recorded step has its counters fixed
+    // either way).
+    const bool general = s->plan.ok && s->g.sz > 1 && s->noise_mode == 0 && s->f[s->plan.phi].noisy &&
+                         recording(s->stream);
+    if (s->path_mode == 0 && s->plan.ok && !general && !hooks_present(s) && fused_noise_ok(s)) {
         // a stale dealiased copy is consumed by one general step first
         if (fused_stale(s)) {
             if (int r = general_steps(s, 1)) return r;

@@ -12,6 +12,8 @@
 namespace cupss {
 
 int fail(int code, const std::string &msg);
+// whether the work enqueued on a stream is being recorded into a graph
+bool recording(hipStream_t stream);
 
 #define HIP_TRY(expr)                                                                                  \
     do {                                                                                               \
