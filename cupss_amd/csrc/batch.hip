@@ -174,7 +174,7 @@ struct FusedBatch {
     std::vector<uint64_t> vgens;  // prefactor-value generations the descriptors hold
 
     // 3D path (the batch of one of a 3D system): h[0] is the descriptor on
-    // the device, twd3 the z-line tile width
+    // the device, twd3 the z-line tile width (kernel_time's name)
     bool d3 = false;
     int twd3 = 0;
 
@@ -1356,44 +1356,6 @@ static int run(FusedBatch &B, int nsteps)
     return settle(B, nsteps);
 }
 
-// z-line tile width of a 3D system: every candidate timed on the system's own
-// buffers.  A z pass in mode 2 reads phi [par] and X_g and writes only the
-// other spectrum buffer, which the next step overwrites: the state is kept.
-static int tune3d(FusedBatch &B, cupss_system s, int par, uint32_t rel)
-{
-    const Geom &g = s->g;
-    const std::vector<int> v = fused3d_z_shapes(g.sz);
-    if (v.empty()) return fail(CUPSS_ERR_UNSUPPORTED, "no z-line tile for this size");
-    hipStream_t st = s->stream;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    float best = 0;
-    int pick = v[0];
-    int rc = CUPSS_OK;
-    for (int w : v) {
-        float ms = 0;
-        hipError_t e = fused3d_z_launch(g.sz, w, B.d, g.nc1, g.sy, par, rel, 2, 0, st);  // warm-up
-        if (e == hipSuccess) e = hipEventRecord(e0, st);
-        for (int r = 0; r < 3 && e == hipSuccess; r++) e = fused3d_z_launch(g.sz, w, B.d, g.nc1, g.sy, par, rel, 2, 0, st);
-        if (e == hipSuccess) e = hipEventRecord(e1, st);
-        if (e == hipSuccess) e = hipEventSynchronize(e1);
-        if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-        if (e != hipSuccess) {
-            rc = fail(CUPSS_ERR_HIP, std::string("z-pass tuning: ") + hipGetErrorString(e));
-            break;
-        }
-        if (w == v[0] || ms < best) {
-            best = ms;
-            pick = w;
-        }
-    }
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
-    if (rc == CUPSS_OK) B.twd3 = pick;
-    return rc;
-}
-
 // The fused step of a 3D system (fused3d.hip), natural layout, no transposes.  A run is
 //   prologue:  z pass in mode 0 and IFFT_y: W_f, Z_f of the current state
 //              (skipped when the previous run left them and nothing changed
@@ -1458,8 +1420,8 @@ static int run3d(FusedBatch &B, cupss_system s, int nsteps)
     const int par0 = F.cur, maxr = a.nreal > 3 ? FUSED_MAX_REAL : (a.nreal > 1 ? 3 : 1);
     const long nrows = (long)g.sy * g.sz;
     hipStream_t st = s->stream;
-    if (!B.twd3)
-        if (int r = tune3d(B, s, par0, rel0)) return r;
+    B.twd3 = fused3d_z_width(g.sz, g.nc1, g.sy);
+    if (!B.twd3) return fail(CUPSS_ERR_UNSUPPORTED, "no z-line tile for this size");
     // the y passes: all products and the noise, all real fields
     const float2 *fin[FUSED_MAX_GROUPS + 1];
     float2 *fout[FUSED_MAX_GROUPS + 1];

@@ -252,15 +252,14 @@ hipError_t fused_ts_reset_launch(unsigned long long *ts, int n, hipStream_t s);
 // A step is four passes: rows (fused3d_rows_launch), FFT_y of X_g and eta
 // (fused3d_y_launch), the z pass (fused3d_z_launch) and IFFT_y of W_f into
 // Z_f (fused3d_y_launch).
-// z-line tile widths (kx lines per workgroup) for sz
-std::vector<int> fused3d_z_shapes(int nz);
+// z-line tile width (kx lines per workgroup) for a box; 0: none
+int fused3d_z_width(int nz, int nc1, int sy);
 hipError_t fused3d_rows_launch(int nc, int maxr, const FusedInst *inst, long nrows, uint32_t step_rel, hipStream_t s);
 // unnormalised C2C transforms (dir) of the y lines kx < ncols[b] of nbuf
 // buffers (at most FUSED_MAX_GROUPS + 1) in one launch; out[b] may be in[b]
 hipError_t fused3d_y_launch(const Geom &g, int dir, int nbuf, const float2 *const *in, float2 *const *out,
                             const int *ncols, hipStream_t s);
-// mode 0: prologue (W_f of the current state), 1: step, 2: step without W_f
-// (timing); herm: phi's kx = 0 and sx/2 planes are not yet Hermitian, project
+// mode 0: prologue (W_f of the current state), 1: step; herm: phi's kx = 0 and sx/2 planes are not yet Hermitian, project
 // them on reading; ts as for fused_cols_launch
 hipError_t fused3d_z_launch(int nz, int twd, const FusedInst *inst, int nc1, int sy, int parity, uint32_t step_rel,
                             int mode, int herm, hipStream_t s, unsigned long long *ts = nullptr);

@@ -409,7 +409,7 @@ __global__ __launch_bounds__((F3zCfg<N, TWD>::THREADS)) __attribute__((amdgpu_wa
 #pragma unroll
         for (int e = 0; e < E; e++) nw[e] = cur[e];
     }
-    if (mode != 2) {
+    {
         // W_f = IFFT_z(mask_f * L_f * phi) on the lines the mask keeps
         const int ny = ky > g.sy / 2 ? ky - g.sy : ky;
         for (int f = 0; f < a.nreal; f++) {
@@ -569,7 +569,7 @@ static std::vector<int> z_shapes()
     return v;
 }
 
-std::vector<int> fused3d_z_shapes(int nz)
+static std::vector<int> fused3d_z_shapes(int nz)
 {
     switch (nz) {
 #define X(N) \
@@ -580,6 +580,22 @@ std::vector<int> fused3d_z_shapes(int nz)
     default:
         return {};
     }
+}
+
+// 16 adjacent lines (128 bytes a row, one cache line) where that still gives
+// two workgroups a CU, else narrower, as in the y passes.  us per step of
+// model B with real-space noise, 16 / 8 / 4 lines where a tile allows them:
+// 64^3 (192 workgroups of 16) 27.5 / 26.9, 32x32x128 27.6 / 26.5 / 25.5,
+// 128x64x64 30.0 / 29.6, 128^3 (640) 48.8 / 50.3 / 49.9, 256^3 219 / 231 / 256.
+// Timing the widths on each new system finds none better than 2 per cent and
+// cost its first run 160 us (32^3) to 850 us (256x256x128), more than the
+// first steps themselves.
+int fused3d_z_width(int nz, int nc1, int sy)
+{
+    int pick = 0;
+    for (int w : fused3d_z_shapes(nz))
+        if (!pick || (w <= 16 && (long)((nc1 + w - 1) / w) * sy >= 512)) pick = w;
+    return pick;
 }
 
 template <int N>
