@@ -461,9 +461,12 @@ static int describe(cupss_system s, FusedInst &a, bool natural = false)
     const FusedPlan &P = s->plan;
     const Geom &g = s->g;
     FieldRec &F = s->f[P.phi];
-    for (size_t i = 0; i < P.real.size(); i++)
+    // 3D: the buffers that the general program has for the same field and term
+    // (a run leaves the dealiased copies unwritten, dstate 2, and the product
+    // transforms live within a step), so that a first run allocates none
+    for (size_t i = 0; i < P.real.size() && !natural; i++)
         if (int r = alloc_spec(&s->fz[i], g)) return r;
-    for (size_t i = 0; i < P.groups.size(); i++)
+    for (size_t i = 0; i < P.groups.size() && !natural; i++)
         if (int r = alloc_spec(&s->fx[i], g)) return r;
     std::memset(&a, 0, sizeof(a));
     a.g = g;
@@ -498,7 +501,7 @@ static int describe(cupss_system s, FusedInst &a, bool natural = false)
         TG.g0 = gi;
         while (gi < (int)P.groups.size() && P.groups[gi].target == f) {
             const FusedGroup &grp = P.groups[gi];
-            a.X[gi] = s->fx[gi];
+            a.X[gi] = natural ? s->t[grp.terms[0]].xhat : s->fx[gi];
             a.pg0[gi] = pi;
             for (size_t q = 0; q < grp.terms.size(); q++) {
                 for (int c : s->t[grp.terms[q]].fac) a.cnt[pi][index_of(P.real, c)]++;
@@ -588,7 +591,7 @@ static int describe(cupss_system s, FusedInst &a, bool natural = false)
         a.p[i] = s->f[f].order;
         a.kmax[i] = a.p[i] > 0 ? std::min(g.nc, g.sx / (a.p[i] + 1)) : g.nc;
         a.kymax[i] = a.p[i] > 0 ? g.sy / (a.p[i] + 1) : g.sy;
-        a.Z[i] = s->fz[i];
+        a.Z[i] = natural ? reinterpret_cast<float2 *>(s->f[f].dreal) : s->fz[i];
         a.zero[i] = step0_zero(s, f) ? 1 : 0;
         a.zsrc[i] = -1;
         a.lbase[i] = -1;
@@ -1373,12 +1376,15 @@ static int run3d(FusedBatch &B, cupss_system s, int nsteps)
     const Geom &g = s->g;
     FusedInst a;
     if (int r = describe(s, a, true)) return r;
-    for (int i = 0; i < a.nreal; i++) {
-        if (!s->fw[i]) {
-            if (int r = alloc_spec(&s->fw[i], g)) return r;
-            HIP_TRY(hipMemsetAsync(s->fw[i], 0, sizeof(float2) * g.nh, s->stream));  // lines off the mask stay zero
-        }
-        a.W[i] = s->fw[i];
+    // W_f lives from a z pass to the y pass after it: in the transform scratch,
+    // the noise and the products, whose lines the z pass has read when it
+    // writes its own; in Z_f itself where there are more real fields (a pass
+    // in place is 1 to 2 per cent of a step slower up to 256x128x128)
+    {
+        std::vector<float2 *> free = {s->scratch};
+        if (a.noise_mode == NOISE_REAL) free.push_back(F.eta);
+        free.insert(free.end(), a.X, a.X + a.ngroups);
+        for (int f = 0; f < a.nreal; f++) a.W[f] = f < (int)free.size() ? free[f] : a.Z[f];
     }
     a.spec[0] = F.spec[0];
     a.spec[1] = F.spec[1];
@@ -1402,17 +1408,22 @@ static int run3d(FusedBatch &B, cupss_system s, int nsteps)
         HIP_TRY(hipStreamSynchronize(s->stream));  // the staging buffer may still feed an earlier copy
         if (B.dcap < 1) {
             hipFree(B.d);
-            hipHostFree(B.pinned);
             B.d = nullptr;
-            B.pinned = nullptr;
-            if (hipMalloc(&B.d, sizeof(FusedInst)) != hipSuccess ||
-                hipHostMalloc(&B.pinned, sizeof(FusedInst)) != hipSuccess)
+            if (hipMalloc(&B.d, sizeof(FusedInst)) != hipSuccess)
                 return fail(CUPSS_ERR_NOMEM, "descriptor allocation failed");
             B.dcap = 1;
         }
-        std::memcpy(B.pinned, &a, sizeof(FusedInst));
-        HIP_TRY(hipMemcpyAsync(B.d, B.pinned, sizeof(FusedInst), hipMemcpyHostToDevice, s->stream));
+        // the first upload from B.h itself: most systems change no more than
+        // the step-0 flags after it, and pinned memory takes 30 to 100 us
         B.h.assign(1, a);
+        const FusedInst *from = B.h.data();
+        if (B.d3) {
+            if (!B.pinned && hipHostMalloc(&B.pinned, sizeof(FusedInst)) != hipSuccess)
+                return fail(CUPSS_ERR_NOMEM, "descriptor allocation failed");
+            std::memcpy(B.pinned, &a, sizeof(FusedInst));
+            from = B.pinned;
+        }
+        HIP_TRY(hipMemcpyAsync(B.d, from, sizeof(FusedInst), hipMemcpyHostToDevice, s->stream));
         B.d3 = true;
     }
     if (!twiddle_sets(s->stream)) return fail(CUPSS_ERR_NOMEM, "twiddle tables");
@@ -1423,27 +1434,17 @@ static int run3d(FusedBatch &B, cupss_system s, int nsteps)
     B.twd3 = fused3d_z_width(g.sz, g.nc1, g.sy);
     if (!B.twd3) return fail(CUPSS_ERR_UNSUPPORTED, "no z-line tile for this size");
     // the y passes: all products and the noise, all real fields
-    const float2 *fin[FUSED_MAX_GROUPS + 1];
-    float2 *fout[FUSED_MAX_GROUPS + 1];
-    int fcols[FUSED_MAX_GROUPS + 1], nf = 0;
-    auto forward = [&](float2 *x) {
-        fin[nf] = x;
-        fout[nf] = x;
-        fcols[nf++] = g.nc1;
+    F3yArgs fwd{}, inv{};
+    auto add = [](F3yArgs &y, const float2 *in, float2 *out, int ncols, int kymax) {
+        y.in[y.n] = in;
+        y.out[y.n] = out;
+        y.ncols[y.n] = ncols;
+        y.kymax[y.n++] = kymax;
     };
-    for (int gi = 0; gi < a.ngroups; gi++) forward(s->fx[gi]);
-    if (a.noise_mode == NOISE_REAL) forward(F.eta);
-    auto inverse_y = [&]() {
-        const float2 *in[FUSED_MAX_REAL];
-        float2 *out[FUSED_MAX_REAL];
-        int cols[FUSED_MAX_REAL];
-        for (int f = 0; f < a.nreal; f++) {
-            in[f] = s->fw[f];
-            out[f] = s->fz[f];
-            cols[f] = a.kmax[f] + 1;
-        }
-        return fused3d_y_launch(g, +1, a.nreal, in, out, cols, st);
-    };
+    for (int gi = 0; gi < a.ngroups; gi++) add(fwd, a.X[gi], a.X[gi], g.nc1, g.sy);
+    if (a.noise_mode == NOISE_REAL) add(fwd, F.eta, F.eta, g.nc1, g.sy);
+    for (int f = 0; f < a.nreal; f++) add(inv, a.W[f], a.Z[f], a.kmax[f] + 1, a.kymax[f]);
+    auto inverse_y = [&]() { return fused3d_y_launch(g, +1, inv, st); };
     // Z_f of the current state: left by the previous run when nothing changed
     // the system since (each run ends with them), else the prologue
     const bool cont = s->cont_step == s->step && s->cont_gen == s->gen;
@@ -1457,9 +1458,9 @@ static int run3d(FusedBatch &B, cupss_system s, int nsteps)
         HIP_TRY(fused_ts_reset_launch(B.pts, FusedBatch::PROF_SLOTS, st));
     }
     for (int i = 0; i < nsteps; i++) {
-        if (nf > 0) {
+        if (fwd.n > 0) {
             HIP_TRY(fused3d_rows_launch(g.nc, maxr, B.d, nrows, rel0 + (uint32_t)i, st));
-            HIP_TRY(fused3d_y_launch(g, -1, nf, fin, fout, fcols, st));
+            HIP_TRY(fused3d_y_launch(g, -1, fwd, st));
         }
         unsigned long long *ts = nullptr;
         if (B.profile && B.pcount < FusedBatch::PROF_SLOTS)

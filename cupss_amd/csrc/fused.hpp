@@ -155,9 +155,9 @@ struct FusedInst {
     float2 *nat;                              // the system's spectrum (natural layout), transform instances
     float2 *cs[FUSED_MAX_CONS][2];            // stored constraints, column-major, like spec
     float2 *cnat[FUSED_MAX_CONS];             // their system buffers (natural layout)
+    float2 *W[FUSED_MAX_REAL];                // 3D: IFFT_z(mask_f * L_f * phi), natural layout
     float2 *Z[FUSED_MAX_REAL];                // IFFT_y(mask_f * field_f), columns kx <= kmax[f]
     float2 *X[FUSED_MAX_GROUPS];              // R2C_x(sum of the products of group g)
-    float2 *W[FUSED_MAX_REAL];                // 3D: IFFT_z(mask_f * L_f * phi), natural layout
     float2 *eta;                              // R2C_x(xi) rows (NOISE_REAL)
     uint64_t step_base;                       // step counter of the first step of a launch sequence
     // row pass
@@ -255,12 +255,21 @@ hipError_t fused_ts_reset_launch(unsigned long long *ts, int n, hipStream_t s);
 // z-line tile width (kx lines per workgroup) for a box; 0: none
 int fused3d_z_width(int nz, int nc1, int sy);
 hipError_t fused3d_rows_launch(int nc, int maxr, const FusedInst *inst, long nrows, uint32_t step_rel, hipStream_t s);
-// unnormalised C2C transforms (dir) of the y lines kx < ncols[b] of nbuf
-// buffers (at most FUSED_MAX_GROUPS + 1) in one launch; out[b] may be in[b]
-hipError_t fused3d_y_launch(const Geom &g, int dir, int nbuf, const float2 *const *in, float2 *const *out,
-                            const int *ncols, hipStream_t s);
-// mode 0: prologue (W_f of the current state), 1: step; herm: phi's kx = 0 and sx/2 planes are not yet Hermitian, project
-// them on reading; ts as for fused_cols_launch
+// unnormalised C2C transforms (dir) of the y lines kx < ncols[b] of n buffers
+// in one launch, out[b] may be in[b]; dir > 0: bins with |ky| > kymax[b] read
+// as zero
+constexpr int F3Y_BUFS = FUSED_MAX_GROUPS + 1;
+static_assert(F3Y_BUFS >= FUSED_MAX_REAL, "a y pass takes the real fields, or the products and the noise");
+struct F3yArgs {
+    const float2 *in[F3Y_BUFS];
+    float2 *out[F3Y_BUFS];
+    int ncols[F3Y_BUFS], kymax[F3Y_BUFS];
+    int n, nc1, sz;
+};
+hipError_t fused3d_y_launch(const Geom &g, int dir, F3yArgs a, hipStream_t s);
+// mode 0: prologue (W_f of the current state), 1: step; herm: phi's kx = 0
+// and sx/2 planes are not yet Hermitian, project them on reading; ts as for
+// fused_cols_launch
 hipError_t fused3d_z_launch(int nz, int twd, const FusedInst *inst, int nc1, int sy, int parity, uint32_t step_rel,
                             int mode, int herm, hipStream_t s, unsigned long long *ts = nullptr);
 // derived fields from phi's spectrum [parity], natural layout

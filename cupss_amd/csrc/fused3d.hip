@@ -24,8 +24,9 @@ namespace cupss {
 //   z     (k_f3z):    X_g, eta -FFT_z-> terms, noise; update of phi
 //                     (setDynamic_k); mask_f * L_f * phi_new -IFFT_z-> W_f
 //   y     (k_f3y):    Z_f = IFFT_y(W_f), lines kx <= kmax_f, in one launch
-// W_f is written only on the (kx, ky) lines the dealias mask of f keeps; the
-// others stay zero from allocation.  The systems have no stored constraint
+// The z pass writes W_f only on the (kx, ky) lines the dealias mask of f
+// keeps; the y pass reads the others as zero.  W_f may be Z_f, or eta or a
+// product transform, of which the z pass reads no line after writing it.  The systems have no stored constraint
 // fields (the host checks).
 
 // Rows of 128 complex points take 8 elements a lane, not the 4 of the 2D tile
@@ -146,13 +147,6 @@ __global__ __launch_bounds__((F3RowCfg<NC, LPB, MAXR>::THREADS)) void k_f3rows(c
 // ones, where one launch for all buffers fills the chip: 128^3 with noise,
 // the two forward transforms 16.4 us in two launches of the general column
 // kernel, 8.8 us here.
-constexpr int F3Y_BUFS = FUSED_MAX_GROUPS + 1;
-struct F3yArgs {
-    const float2 *in[F3Y_BUFS];
-    float2 *out[F3Y_BUFS];
-    int ncols[F3Y_BUFS];
-    int nc1, sz;
-};
 template <int N, int TWD>
 struct F3yCfg {
     static constexpr int E = N >= 4096 ? 16 : (N >= 8 ? 8 : N);
@@ -180,10 +174,21 @@ __global__ __launch_bounds__((F3yCfg<N, TWD>::THREADS)) void k_f3y(F3yArgs a, co
     StageTwiddles<N, E, C::THREADS> twl;
     twl.load(sets);
     const float2 *in = a.in[blockIdx.y];
+    const int kymax = a.kymax[blockIdx.y];
     float2 v[E];
 #pragma unroll
-    for (int e = 0; e < E; e++)
-        v[e] = active ? gload(in, base + (long)(t + e * T) * nc1) : make_float2(0.f, 0.f);
+    for (int e = 0; e < E; e++) {
+        // dir > 0: only the bins of the dealias mask hold the field; the
+        // others load the lane's first bin again, so that one branch covers
+        // all loads
+        const bool keep = DIR < 0 || min(t + e * T, N - (t + e * T)) <= kymax;
+        v[e] = active ? gload(in, base + t * nc1 + (keep ? e * T * nc1 : 0)) : make_float2(0.f, 0.f);
+    }
+    if constexpr (DIR > 0) {
+#pragma unroll
+        for (int e = 0; e < E; e++)
+            if (min(t + e * T, N - (t + e * T)) > kymax) v[e] = make_float2(0.f, 0.f);
+    }
     twl.store(tst, sets);
     __syncthreads();
     fft_line<N, E, DIR, TW_STAGE, false, WL>(v, lds + c * C::LL, t, tst);
@@ -409,33 +414,31 @@ __global__ __launch_bounds__((F3zCfg<N, TWD>::THREADS)) __attribute__((amdgpu_wa
 #pragma unroll
         for (int e = 0; e < E; e++) nw[e] = cur[e];
     }
-    {
-        // W_f = IFFT_z(mask_f * L_f * phi) on the lines the mask keeps
-        const int ny = ky > g.sy / 2 ? ky - g.sy : ky;
-        for (int f = 0; f < a.nreal; f++) {
-            if (kx0 > a.kmax[f] || abs(ny) > a.kymax[f]) continue;  // uniform over the workgroup
-            const int lz = a.p[f] > 0 ? g.sz / (a.p[f] + 1) : g.sz;
-            const bool zero = !upd && a.zero[f] != 0;
-            float2 v[E];
-            const TermRefDev &LM = a.lmul[f];
-            float lm[E];
-            if (LM.npres > 0) multiplier_line<E>(a.pool, LM.pres0, LM.npres, LM.mult_i, lb, lm);
+    // W_f = IFFT_z(mask_f * L_f * phi) on the lines the mask keeps
+    const int ny = ky > g.sy / 2 ? ky - g.sy : ky;
+    for (int f = 0; f < a.nreal; f++) {
+        if (kx0 > a.kmax[f] || abs(ny) > a.kymax[f]) continue;  // uniform over the workgroup
+        const int lz = a.p[f] > 0 ? g.sz / (a.p[f] + 1) : g.sz;
+        const bool zero = !upd && a.zero[f] != 0;
+        float2 v[E];
+        const TermRefDev &LM = a.lmul[f];
+        float lm[E];
+        if (LM.npres > 0) multiplier_line<E>(a.pool, LM.pres0, LM.npres, LM.mult_i, lb, lm);
 #pragma unroll
-            for (int e = 0; e < E; e++) {
-                const int kz = t + e * T;
-                const int nz = kz > g.sz / 2 ? kz - g.sz : kz;
-                const bool keep = !zero && kx <= a.kmax[f] && abs(nz) <= lz;
-                const float2 w = LM.npres > 0 ? apply_mult(lm[e], LM.mult_i, nw[e]) : nw[e];
-                v[e] = keep ? w : make_float2(0.f, 0.f);
-            }
-            fft_line<N, E, +1, TW_STAGE, false, (TWD * T <= 64)>(v, L, t, tws);
-            if (active && kx <= a.kmax[f]) {
-                float2 *__restrict__ w = a.W[f];
-#pragma unroll
-                for (int e = 0; e < E; e++) gstore(w, base + (long)(t + e * T) * plane, v[e]);
-            }
-            line_sync<(TWD * T <= 64)>();
+        for (int e = 0; e < E; e++) {
+            const int kz = t + e * T;
+            const int nz = kz > g.sz / 2 ? kz - g.sz : kz;
+            const bool keep = !zero && kx <= a.kmax[f] && abs(nz) <= lz;
+            const float2 w = LM.npres > 0 ? apply_mult(lm[e], LM.mult_i, nw[e]) : nw[e];
+            v[e] = keep ? w : make_float2(0.f, 0.f);
         }
+        fft_line<N, E, +1, TW_STAGE, false, (TWD * T <= 64)>(v, L, t, tws);
+        if (active && kx <= a.kmax[f]) {
+            float2 *__restrict__ w = a.W[f];
+#pragma unroll
+            for (int e = 0; e < E; e++) gstore(w, base + (long)(t + e * T) * plane, v[e]);
+        }
+        line_sync<(TWD * T <= 64)>();
     }
     if (slot) {
         __syncthreads();
@@ -501,23 +504,23 @@ hipError_t fused3d_rows_launch(int nc, int maxr, const FusedInst *inst, long nro
 #define F3Y_TWD(X) X(1) X(2) X(4) X(8) X(16) X(32) X(64)
 
 template <int N>
-static hipError_t f3y_n(int dir, const F3yArgs &a, int nbuf, hipStream_t s, const float2 *sets)
+static hipError_t f3y_n(int dir, const F3yArgs &a, hipStream_t s, const float2 *sets)
 {
     int most = 1;
-    for (int b = 0; b < nbuf; b++) most = std::max(most, a.ncols[b]);
+    for (int b = 0; b < a.n; b++) most = std::max(most, a.ncols[b]);
     // 16 adjacent lines (128 bytes a row, one cache line) where that still
     // gives two workgroups a CU, else narrower: 128^3, two buffers, 16 lines
     // 8.8 us against 16.4 us for 4 lines of a buffer at a time
     int pick = 0;
 #define X(TWD)                                                                                              \
     if constexpr (F3yCfg<N, TWD>::valid())                                                                  \
-        if (!pick || (TWD <= 16 && (long)((most + TWD - 1) / TWD) * a.sz * nbuf >= 512)) pick = TWD;
+        if (!pick || (TWD <= 16 && (long)((most + TWD - 1) / TWD) * a.sz * a.n >= 512)) pick = TWD;
     F3Y_TWD(X)
 #undef X
 #define X(TWD)                                                                                              \
     if constexpr (F3yCfg<N, TWD>::valid())                                                                  \
         if (pick == TWD) {                                                                                  \
-            const dim3 grid((unsigned)xcd_blocks((long)((most + TWD - 1) / TWD) * a.sz), (unsigned)nbuf);   \
+            const dim3 grid((unsigned)xcd_blocks((long)((most + TWD - 1) / TWD) * a.sz), (unsigned)a.n);   \
             if (dir < 0)                                                                                    \
                 hipLaunchKernelGGL((k_f3y<N, TWD, -1>), grid, dim3(F3yCfg<N, TWD>::THREADS), 0, s, a, sets); \
             else                                                                                            \
@@ -529,25 +532,18 @@ static hipError_t f3y_n(int dir, const F3yArgs &a, int nbuf, hipStream_t s, cons
     return hipErrorInvalidValue;
 }
 
-hipError_t fused3d_y_launch(const Geom &g, int dir, int nbuf, const float2 *const *in, float2 *const *out,
-                            const int *ncols, hipStream_t s)
+hipError_t fused3d_y_launch(const Geom &g, int dir, F3yArgs a, hipStream_t s)
 {
     const float2 *sets = twiddle_sets(s);
     if (!sets) return hipErrorOutOfMemory;
-    if (nbuf <= 0) return hipSuccess;
-    if (nbuf > F3Y_BUFS) return hipErrorInvalidValue;
-    F3yArgs a{};
-    for (int b = 0; b < nbuf; b++) {
-        a.in[b] = in[b];
-        a.out[b] = out[b];
-        a.ncols[b] = ncols[b];
-    }
+    if (a.n <= 0) return hipSuccess;
+    if (a.n > F3Y_BUFS) return hipErrorInvalidValue;
     a.nc1 = g.nc1;
     a.sz = g.sz;
     switch (g.sy) {
 #define X(N) \
     case N:  \
-        return f3y_n<N>(dir, a, nbuf, s, sets);
+        return f3y_n<N>(dir, a, s, sets);
         F3Y_CASES(X)
 #undef X
     default:
@@ -583,18 +579,22 @@ static std::vector<int> fused3d_z_shapes(int nz)
 }
 
 // 16 adjacent lines (128 bytes a row, one cache line) where that still gives
-// two workgroups a CU, else narrower, as in the y passes.  us per step of
-// model B with real-space noise, 16 / 8 / 4 lines where a tile allows them:
-// 64^3 (192 workgroups of 16) 27.5 / 26.9, 32x32x128 27.6 / 26.5 / 25.5,
-// 128x64x64 30.0 / 29.6, 128^3 (640) 48.8 / 50.3 / 49.9, 256^3 219 / 231 / 256.
-// Timing the widths on each new system finds none better than 2 per cent and
-// cost its first run 160 us (32^3) to 850 us (256x256x128), more than the
-// first steps themselves.
+// two workgroups a CU and leaves no more than a fifth of the lanes without a
+// line (33 bins: 15 of 48), else narrower.  us per step of model B with
+// real-space noise, 16 / 8 / 4 lines where a tile allows them: 64^3 (192
+// workgroups of 16) 27.5 / 26.9, 32x32x128 27.6 / 26.5 / 25.5, 128x64x64
+// 30.0 / 29.6, 128^3 (640) 48.1 / 48.6 / 49.3, 64x256x256 80.5 / 77.1 / 77.6,
+// 256x128x128 70.3 / 72.2 / 69.3, 256x256x128 111 / 120 / 114, 256^3
+// 219 / 231 / 256.  Timing the widths on each new system finds none better
+// than 2 per cent and cost its first run 160 us (32^3) to 850 us (256x256x128),
+// more than the first steps themselves.
 int fused3d_z_width(int nz, int nc1, int sy)
 {
     int pick = 0;
-    for (int w : fused3d_z_shapes(nz))
-        if (!pick || (w <= 16 && (long)((nc1 + w - 1) / w) * sy >= 512)) pick = w;
+    for (int w : fused3d_z_shapes(nz)) {
+        const int tiles = (nc1 + w - 1) / w;
+        if (!pick || (w <= 16 && (long)tiles * sy >= 512 && 4 * tiles * w <= 5 * nc1)) pick = w;
+    }
     return pick;
 }
 

@@ -128,7 +128,6 @@ extern "C" int cupss_system_destroy(cupss_system s)
     for (auto *p : s->fz) hipFree(p);
     for (auto *p : s->fx) hipFree(p);
     for (auto *p : s->ft) hipFree(p);
-    for (auto *p : s->fw) hipFree(p);
     for (auto &c : s->fc) {
         hipFree(c[0]);
         hipFree(c[1]);
@@ -320,8 +319,15 @@ extern "C" int cupss_field_get_dealiased(cupss_system s, int field, float *host)
         std::memset(host, 0, sizeof(float) * s->g.n);
         return CUPSS_OK;
     }
-    if (int r = materialize(s, field)) return r;
-    HIP_TRY(hipMemcpyAsync(host, F.dreal, sizeof(float) * s->g.n, hipMemcpyDeviceToHost, s->stream));
+    const float *src = F.dreal;
+    if (s->g.sz > 1 && F.dstate == 2) {
+        // dreal holds what the next fused run goes on from (run3d)
+        HIP_TRY(c2r(s->g, F.spec[F.cur], F.order, 1.0f / (float)s->g.n, s->rtmp, s->scratch, s->stream));
+        src = s->rtmp;
+    } else if (int r = materialize(s, field)) {
+        return r;
+    }
+    HIP_TRY(hipMemcpyAsync(host, src, sizeof(float) * s->g.n, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     return CUPSS_OK;
 }
@@ -358,6 +364,11 @@ extern "C" int cupss_field_spectrum_device(cupss_system s, int field, void **dev
     return CUPSS_OK;
 }
 
+static size_t dreal_bytes(const Geom &g)
+{
+    return g.sz > 1 ? sizeof(float2) * (size_t)g.nh : sizeof(float) * (size_t)g.n;
+}
+
 extern "C" int cupss_system_prepare(cupss_system s)
 {
     if (int r = check_sys(s)) return r;
@@ -373,7 +384,7 @@ extern "C" int cupss_system_prepare(cupss_system s)
             }
     for (auto &F : s->f) {
         if (F.order > 0 && !F.dreal) {
-            if (hipMalloc(&F.dreal, sizeof(float) * s->g.n) != hipSuccess)
+            if (hipMalloc(&F.dreal, dreal_bytes(s->g)) != hipSuccess)
                 return fail(CUPSS_ERR_NOMEM, "device allocation failed");
             // zero until the field's first update (the reference's step-0 state)
             HIP_TRY(hipMemsetAsync(F.dreal, 0, sizeof(float) * s->g.n, s->stream));
@@ -835,14 +846,12 @@ extern "C" int cupss_system_device_bytes(cupss_system s, size_t *bytes)
     if (s->full) b += sizeof(float2) * (size_t)s->g.n;
     for (auto &F : s->f) {
         b += 2 * spec;
-        if (F.dreal) b += real;
+        if (F.dreal) b += dreal_bytes(s->g);
         if (F.eta) b += spec;
     }
     for (auto &T : s->t)
         if (T.xhat) b += spec;
-    if (s->plan.ok && s->g.sz > 1)  // the 3D fused path's buffers (Z_f, W_f, X_g)
-        b += spec * (2 * s->plan.real.size() + s->plan.groups.size());
-    else if (s->plan.ok)  // the fused path's buffers, allocated at its first run
+    if (s->plan.ok && s->g.sz == 1)  // the fused path's buffers, allocated at its first run
         b += spec * (2 + 2 * s->plan.cons.size() + s->plan.real.size() + s->plan.groups.size()) + fused_table_bytes(s);
     b += line_device_bytes(s);
     *bytes = b;

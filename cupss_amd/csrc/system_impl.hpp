@@ -32,6 +32,7 @@ struct FieldRec {
     int order = 0;  // dealias order, 0 = none
     float2 *spec[2] = {nullptr, nullptr};
     int cur = 0;
+    // N floats; 3D: nh float2, where fused runs keep the field's Z_f
     float *dreal = nullptr;
     // dealiased real copy: 0 = zero (never updated, the reference's step-0
     // state), 1 = dreal holds C2R(mask*spec), 2 = same but not yet written
@@ -93,6 +94,7 @@ struct cupss_system_t {
     int path_mode = 0;        // 0 = fused step when eligible, 1 = general step only
     int noise_mode = 0;       // 0 = real-space Philox + R2C, 1 = spectral-space Philox
     cupss::FusedPlan plan;
+    // 2D fused path's real fields and products (3D: FieldRec::dreal, TermRec::xhat)
     float2 *fz[cupss::FUSED_MAX_REAL] = {};
     float2 *fx[cupss::FUSED_MAX_GROUPS] = {};
     float2 *ft[2] = {nullptr, nullptr};  // phi's spectrum, column-major, during fused runs
@@ -102,7 +104,6 @@ struct cupss_system_t {
     float *ftab = nullptr;
     int ftab_n = 0;
     uint64_t ftab_gen = 0, ftab_vgen = 0;
-    float2 *fw[cupss::FUSED_MAX_REAL] = {};     // 3D: IFFT_z of the masked real fields (zero off the kept lines)
     // After a fused run, fc[.][cont_buf] holds the stored fields' values of
     // the next step's phase A/B; a run that starts at step cont_step with
     // generation cont_gen continues from them.  Anything that changes the
