@@ -736,7 +736,9 @@ static int class_tables(const FusedBatch &B, const FusedBatch::Class &c, int lpb
 }
 
 // shapes before (or without) tuning: up to 8 rows per row workgroup, up to
-// 256 threads per column workgroup
+// 256 threads per column workgroup (512 with the 4 elements a lane of 256- and
+// 1024-point columns: 16 KPZ systems of 256^2 21.9 us a step against 19.9,
+// 4 of model H 1024^2 172 against 149)
 static void default_shapes(FusedBatch::Class &c)
 {
     const std::vector<int> rs = fused_row_shapes(c.nc, c.ny, c.width), cs = fused_col_shapes(c.ny);
@@ -744,9 +746,8 @@ static void default_shapes(FusedBatch::Class &c)
     for (int v : rs)
         if (v <= 8) c.lpb = v;
     c.twd = cs.empty() ? 0 : cs.front();
-    const int T = c.ny >= 4096 ? c.ny / 16 : (c.ny >= 8 ? c.ny / 8 : 1);
     for (int v : cs)
-        if (v * T <= 256) c.twd = v;
+        if (v * fused_col_lanes(c.ny) <= 256) c.twd = v;
 }
 
 static int build(FusedBatch &B)

@@ -450,6 +450,19 @@ std::vector<int> fused_col_shapes(int ny)
     }
 }
 
+int fused_col_lanes(int ny)
+{
+    switch (ny) {
+#define X(N) \
+    case N:  \
+        return FColCfg<N, 1>::T;
+        FUSED_COL_CASES(X)
+#undef X
+    default:
+        return 0;
+    }
+}
+
 template <int NC, int MAXR>
 static hipError_t frows_n(int lpb, const FusedInst *inst, const FusedBlock *blocks, int nblocks, uint32_t step_rel,
                           hipStream_t s, const float2 *sets)

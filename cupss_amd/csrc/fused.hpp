@@ -219,6 +219,8 @@ bool fused_shapes_exist(int sx, int sy, int sz, int nreal);
 int fused_row_width(int nreal);
 std::vector<int> fused_row_shapes(int nc, int ny, int width);
 std::vector<int> fused_col_shapes(int ny);
+// lanes of one column (0: no column kernel)
+int fused_col_lanes(int ny);
 
 hipError_t fused_rows_launch(int nc, int lpb, int width, const FusedInst *inst, const FusedBlock *blocks,
                              int nblocks, uint32_t step_rel, hipStream_t s);

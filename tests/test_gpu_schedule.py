@@ -1,0 +1,36 @@
+"""The tiles that a batch's size classes take without timing runs."""
+import re
+
+import pytest
+
+import cupss_amd as C
+from tests.helpers import build_system, spec_cahn_hilliard, spec_kpz
+from cupss_amd.systems import spec_gray_scott
+
+pytestmark = pytest.mark.gpu
+
+
+def tiles(specs, autotune):
+    """(rows, columns) a workgroup of each size class after a run."""
+    b = C.Batch(autotune=autotune)
+    keep = [build_system(C.System, C.pres, spec)[0] for spec in specs]
+    for s in keep:
+        b.add(s)
+    b.step(2)
+    b.synchronize()
+    got = [(int(m.group(1)), int(m.group(2)))
+           for m in re.finditer(r"rows/wg (\d+), cols/wg (\d+)", b.schedule())]
+    b.close()
+    for s in keep:
+        s.close()
+    return got
+
+
+# lanes of a column: the points by the elements a lane holds (8; 4 for 256 and
+# from 1024 on; 16 at 4096)
+@pytest.mark.parametrize("ny,lanes", [(8, 1), (32, 4), (64, 8), (256, 64), (512, 64), (1024, 256), (2048, 512),
+                                      (4096, 256)])
+def test_default_columns_keep_256_threads(ny, lanes):
+    (rows, cols), = tiles([spec_cahn_hilliard((32, ny, 1))], False)
+    assert rows == 8
+    assert cols == max([1] + [c for c in (1, 2, 4, 8, 16) if c * lanes <= 256])
