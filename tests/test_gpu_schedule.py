@@ -34,3 +34,10 @@ def test_default_columns_keep_256_threads(ny, lanes):
     (rows, cols), = tiles([spec_cahn_hilliard((32, ny, 1))], False)
     assert rows == 8
     assert cols == max([1] + [c for c in (1, 2, 4, 8, 16) if c * lanes <= 256])
+
+
+@pytest.mark.parametrize("autotune", [True, False])
+@pytest.mark.parametrize("members", [1, 5])
+def test_128_square_takes_fixed_tiles(members, autotune):
+    mixed = [spec_kpz(128), spec_gray_scott(128)]
+    assert tiles([spec_cahn_hilliard((128, 128, 1))] * members + mixed, autotune) == [(4, 2)] * 2
