@@ -876,7 +876,7 @@ static int refresh(FusedBatch &B)
 {
     const size_t n = B.h.size();
     if (B.dirty.size() != n) B.dirty.assign(n, 1);
-    bool any = false;
+    bool any = false, all = true;
     for (size_t i = 0; i < n; i++) {
         if (B.vgens[i] != B.sys[i]->vgen) {  // new prefactor values, same structure: new pool
             if (int r = describe(B.sys[i], B.h[i])) return r;
@@ -886,9 +886,13 @@ static int refresh(FusedBatch &B)
         }
         if (run_view(B.sys[i], B.is_elem[i], B.h[i])) B.dirty[i] = 1;
         any = any || B.dirty[i];
+        all = all && B.dirty[i];
     }
     if (!any) return CUPSS_OK;
-    if (int r = catch_up(B)) return r;
+    if (all)
+        B.lag = 0;  // every descriptor is uploaded, as of now
+    else if (int r = catch_up(B))
+        return r;
     if (B.staged) HIP_TRY(hipEventSynchronize(B.staged));
     for (size_t i = 0; i < n;) {
         if (!B.dirty[i]) {
@@ -1243,11 +1247,9 @@ static int flush(FusedBatch &B)
 {
     if (!B.settle_pending) return CUPSS_OK;
     B.settle_pending = false;
-    // with the counters caught up, the final state is in buffer [0] and the
-    // last step's start in [1]
-    if (B.ntb > 0)
-        if (int r = catch_up(B)) return r;
-    if (B.ntb > 0) HIP_TRY(fused_settle_launch(B.d, B.tb, B.ntb, 0, B.stream));
+    // the final state is `lag` steps after the descriptors', the last step's
+    // start in the other buffer
+    if (B.ntb > 0) HIP_TRY(fused_settle_launch(B.d, B.tb, B.ntb, (int)(B.lag & 1), B.stream));
     bool waits = false;
     for (cupss_system s : B.sys) {
         if (s->pending == &B) s->pending = nullptr;
