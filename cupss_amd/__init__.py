@@ -67,6 +67,7 @@ _SIGS = {
     "cupss_system_set_dt": (_I, [_VP, _F]),
     "cupss_system_set_path": (_I, [_VP, _I]),
     "cupss_system_fused_eligible": (_I, [_VP]),
+    "cupss_system_stat": (_I, [_VP, ctypes.c_char_p, ctypes.POINTER(ctypes.c_long)]),
     "cupss_system_set_noise_mode": (_I, [_VP, _I]),
     "cupss_batch_create": (_I, [_VP, ctypes.POINTER(_VP)]),
     "cupss_batch_destroy": (_I, [_VP]),
@@ -222,6 +223,12 @@ class System:
         ms, pts, name = ctypes.c_float(), ctypes.c_double(), ctypes.create_string_buffer(64)
         check(self.L.cupss_system_kernel_time(self.h, ctypes.byref(ms), ctypes.byref(pts), name, 64))
         return ms.value, pts.value, name.value.decode()
+
+    def stat(self, name):
+        """A count of the system's work: "fused_steps", "line_steps", "line_plans"."""
+        v = ctypes.c_long()
+        check(self.L.cupss_system_stat(self.h, name.encode(), ctypes.byref(v)))
+        return v.value
 
     def device_bytes(self):
         b = ctypes.c_size_t()

@@ -7,10 +7,11 @@
 // general program takes seven launches for a step of a KPZ line, 27 us of
 // which nearly all is launch and first-access latency.  Here every field's
 // spectrum, the dealiased copies, the product transforms and the noise stay
-// in LDS for the whole run, one wavefront takes one transform (independent
-// transforms run side by side on different wavefronts, the draws of the next
-// step on those left over), and the stages of a step are separated by
-// workgroup barriers.  What bounds it is the chain of a step: an inverse and
+// in LDS for the whole run, and the stages of a step are separated by
+// workgroup barriers.  Up to 512 complex points one wavefront takes one
+// transform (independent transforms run side by side on different wavefronts,
+// the draws of the next step on those left over); longer ones take all of the
+// workgroup's, one after another (LineCfg).  What bounds it is the chain of a step: an inverse and
 // a forward transform of about 1.6 us each and two updates of 0.9 us, mostly
 // LDS and scalar-load latency.  Measured, us per step of a KPZ line with
 // real-space noise, general program -> here: 64 points 28 -> 3.5, 256 points
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(LineCfg<NC>::THREADS) void k_line(const LineProg *_
                     v[e] = cadd(cadd(A, Bc), mul_i<+1>(xo));
                 }
                 fft_line<NC, E, +1, TW_STAGE, false, WL>(v, L, t, tws);
-                                if (on) {
+                if (on) {
 #pragma unroll
                     for (int e = 0; e < E; e++) dreal[F.dslot * NC + t + e * T] = cscale(v[e], scale);
                 }
@@ -412,7 +413,8 @@ __global__ __launch_bounds__(256) void k_line_tables(UpdateArgs a, float *__rest
 // ------------------------------------------------------------ host
 
 struct LineState {
-    uint64_t gen = 0, vgen = 0;  // the program and prefactor values it was made for
+    uint64_t gen = 0, vgen = 0;    // the program and prefactor values the device holds
+    uint64_t pgen = 0, pvgen = 0;  // those it was laid out for, whether it fits or not
     bool ok = false;
     long bytes = 0;              // dynamic LDS
     bool tab = false;            // the multiplier tables fit it too
@@ -458,7 +460,9 @@ static long line_bytes(const LineProg &p, bool tables)
 
 // The program of a 1D system, or ok = false where it does not fit one
 // workgroup: more fields or terms than the descriptor holds, or more LDS than
-// one workgroup has (about six fields on 4096 points).
+// one workgroup has.  On 4096 points two fields with one dealiased copy, one
+// product and real-space noise (a KPZ line) take 149568 of the 153600 bytes;
+// on 2048 twice that fits (140408).
 static void line_plan(cupss_system s, LineState &S)
 {
     S.ok = false;
@@ -539,16 +543,17 @@ bool line_eligible(cupss_system s)
         S = new LineState();
         s->line = S;
     }
-    if (S->gen != s->gen || S->vgen != s->vgen) {
+    if (S->pgen != s->gen || S->pvgen != s->vgen) {
         line_plan(s, *S);
-        if (S->ok) {
-            // the upload cannot be recorded into a graph: a caller's capture
-            // that starts before the program was uploaded records the general
-            // program's launches
-            if (recording(s->stream)) return false;
-        }
+        S->pgen = s->gen;
+        S->pvgen = s->vgen;
+        s->line_plans++;
     }
-    return S->ok;
+    if (!S->ok) return false;
+    // the upload cannot be recorded into a graph: a caller's capture that
+    // starts before the program was uploaded records the general program's
+    // launches
+    return (S->gen == s->gen && S->vgen == s->vgen) || !recording(s->stream);
 }
 
 template <int NC, bool TAB>
@@ -628,6 +633,7 @@ int line_steps(cupss_system s, int nsteps)
             if (F.order > 0) F.dstate = 1;
         }
         s->step += (uint64_t)k;
+        s->line_steps += k;
         done += k;
     }
     return CUPSS_OK;

@@ -837,6 +837,21 @@ extern "C" int cupss_system_kernel_time(cupss_system s, float *avg_ms, double *p
     return fused_kernel_time(s, avg_ms, points, name, len);
 }
 
+extern "C" int cupss_system_stat(cupss_system s, const char *name, long *value)
+{
+    if (int r = check_sys(s)) return r;
+    if (!name || !value) return fail(CUPSS_ERR_INVALID, "null name or value");
+    if (std::strcmp(name, "fused_steps") == 0)
+        *value = s->fused_steps;
+    else if (std::strcmp(name, "line_steps") == 0)
+        *value = s->line_steps;
+    else if (std::strcmp(name, "line_plans") == 0)
+        *value = s->line_plans;
+    else
+        return fail(CUPSS_ERR_INVALID, "no such count");
+    return CUPSS_OK;
+}
+
 extern "C" int cupss_system_device_bytes(cupss_system s, size_t *bytes)
 {
     if (int r = check_sys(s)) return r;

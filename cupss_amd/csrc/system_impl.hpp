@@ -117,7 +117,9 @@ struct cupss_system_t {
     // generation cont_gen resumes from them (no transpose in, no prologue)
     int cont_ft = 0;
     bool resume_now = false;
-    long fused_steps = 0;     // steps taken by the fused path (diagnostics)
+    // cupss_system_stat: steps by the fused path and by the 1D kernel, layouts
+    // of the 1D program
+    long fused_steps = 0, line_steps = 0, line_plans = 0;
     uint64_t step = 0;
     int device = 0;
     void *batch = nullptr;    // internal one-instance fused batch

@@ -172,6 +172,11 @@ int cupss_system_set_noise_mode(cupss_system s, int mode);
 /* 1 if cupss_system_advance would take the fused 2D step (and
  * cupss_batch_add accept the system) */
 int cupss_system_fused_eligible(cupss_system s);
+/* a count of the system's work so far, by name: "fused_steps" (the fused 2D
+ * and 3D steps, in batches too), "line_steps" (the 1D steps in one
+ * workgroup; the other steps of a system are the general program's) and
+ * "line_plans" (how often the 1D program was laid out) */
+int cupss_system_stat(cupss_system s, const char *name, long *value);
 /* 0 = direct launches (default); K (even, >= 2) = runs of at least K steps
  * replay K steps from a hipGraph captured at the first such run.  Applies
  * to the fused path and to the general step program of noiseless systems
