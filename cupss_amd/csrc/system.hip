@@ -773,10 +773,11 @@ static int general_advance(cupss_system s, int nsteps)
 }
 
 
-// The fused 3D step takes either noise draw.  With the real-space one it
-// starts at 32^3 points (25 us a step against 36 of the general program
-// there, 49 against 91 at 128^3): on smaller boxes both are a chain of
-// launches, and the results keep the general program's bits.
+// The fused 3D step takes either noise draw, the real-space one from 32^3
+// points on.  It is the faster one below as well (us a step, fused / general:
+// 16x8x8 21.7 / 31.5, 16^3 23.5 / 34.4, 32x32x16 23.0 / 35.6, 32^3 23.6 /
+// 36.1, 128^3 48 / 91), but there both are a chain of short launches, and
+// small boxes keep the general program's bits, which programs compare.
 bool cupss::fused_noise_ok(cupss_system s)
 {
     if (!s->plan.ok || s->noise_mode == 1) return true;
