@@ -1712,7 +1712,9 @@ static int kernel_time(FusedBatch &B, float *avg_ms, double *points, char *name,
     for (int i : c.insts) pts += (double)B.h[i].g.n;
     if (points) *points = pts;
     if (name && len > 0) {
-        if (c.small)
+        if (c.small && c.lean)
+            std::snprintf(name, (size_t)len, "k_fsmall<%d, %d>", c.nc, c.ny);
+        else if (c.small)
             std::snprintf(name, (size_t)len, "k_fsmall<%d, %d, %s, %s>", c.nc, c.ny, c.cons ? "true" : "false",
                           c.cons == 2 ? "true" : "false");
         else if (c.lean)

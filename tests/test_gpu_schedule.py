@@ -41,3 +41,14 @@ def test_default_columns_keep_256_threads(ny, lanes):
 def test_128_square_takes_fixed_tiles(members, autotune):
     mixed = [spec_kpz(128), spec_gray_scott(128)]
     assert tiles([spec_cahn_hilliard((128, 128, 1))] * members + mixed, autotune) == [(4, 2)] * 2
+
+
+@pytest.mark.parametrize("spec,name", [
+    (spec_kpz(64), "k_fsmall<32, 64>"), (spec_gray_scott(64), "k_fsmall<32, 64, true, true>"),
+    (spec_kpz(128), "k_fcols<128, 2>"), (spec_gray_scott(128), "k_fcols<128, 2, true, true>")])
+def test_timed_kernel_is_the_one_launched(spec, name):
+    """Simple systems run the lean kernels, which have no template flags."""
+    s, _ = build_system(C.System, C.pres, spec)
+    s.profile_kernel(True)
+    s.step(4)
+    assert s.kernel_time()[2] == name
