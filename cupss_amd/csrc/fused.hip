@@ -46,19 +46,19 @@ namespace cupss {
 
 // ------------------------------------------------------------ row and column kernels
 
-template <int NC, int LPB, int MAXR>
-__global__ __launch_bounds__((FRowCfg<NC, LPB, MAXR>::THREADS)) void k_frows(const FusedInst *__restrict__ insts,
+template <int NC, int LPB, int MAXR, bool SINGLE>
+__global__ __launch_bounds__((FRowCfg<NC, LPB, MAXR, SINGLE>::THREADS)) void k_frows(const FusedInst *__restrict__ insts,
                                                                           const FusedBlock *__restrict__ blocks,
                                                                           uint32_t step_rel,
                                                                           const float2 *__restrict__ sets)
 {
-    using C = FRowCfg<NC, LPB, MAXR>;
+    using C = FRowCfg<NC, LPB, MAXR, SINGLE>;
     __shared__ __align__(16) float2 tws[2 * NC];
     __shared__ __align__(16) float2 tst[tw_stage_alloc(NC, C::E)];
     __shared__ float2 tile[C::LEN];
     const FusedBlock blk = blocks[blockIdx.x];
     if (blk.inst < 0) return;
-    frows_tile<NC, LPB, MAXR>(insts[blk.inst], blk.line, step_rel, sets, true, tws, tst, tile);
+    frows_tile<NC, LPB, MAXR, SINGLE>(insts[blk.inst], blk.line, step_rel, sets, true, tws, tst, tile);
 }
 
 template <int N, int TWD, bool CONS, bool XDYN>
@@ -463,20 +463,33 @@ int fused_col_lanes(int ny)
     }
 }
 
+// Rows of 256 and 512 complex points: pairs (FRowCfg::PAIR) up to 4096 rows a
+// launch, beyond that their LDS and registers cost more than the latency they
+// hide.  us per step, singly / pairs: Gray-Scott 512^2 x8 (4096 rows) 36.4 /
+// 35.6, x16 53.4 / 56.0, x32 97 / 100; a three-field system 512^2 x8 31.5 /
+// 31.0, x16 45.1 / 48.1, 1024^2 x4 (4096 rows) 59.7 / 59.8, x8 93 / 100.
+constexpr long ROW_PAIRS_MAX = 4096;
 template <int NC, int MAXR>
 static hipError_t frows_n(int lpb, const FusedInst *inst, const FusedBlock *blocks, int nblocks, uint32_t step_rel,
                           hipStream_t s, const float2 *sets)
 {
-#define X(LPB)                                                                                                   \
-    if constexpr (FRowCfg<NC, LPB, MAXR>::valid()) {                                                            \
-        if (lpb == LPB) {                                                                                        \
-            hipLaunchKernelGGL((k_frows<NC, LPB, MAXR>), dim3(nblocks), dim3(FRowCfg<NC, LPB, MAXR>::THREADS), 0, \
-                               s, inst, blocks, step_rel, sets);                                                 \
-            return hipGetLastError();                                                                            \
-        }                                                                                                        \
+    constexpr bool BOTH = NC >= 256 && FRowCfg<NC, 1, MAXR>::PAIR;
+#define L(LPB, SINGLE)                                                                                    \
+    hipLaunchKernelGGL((k_frows<NC, LPB, MAXR, SINGLE>), dim3(nblocks),                                  \
+                       dim3(FRowCfg<NC, LPB, MAXR, SINGLE>::THREADS), 0, s, inst, blocks, step_rel, sets)
+#define X(LPB)                                                           \
+    if constexpr (FRowCfg<NC, LPB, MAXR>::valid()) {                    \
+        if (lpb == LPB) {                                                \
+            if (BOTH && (long)nblocks * LPB > ROW_PAIRS_MAX)             \
+                L(LPB, BOTH);                                            \
+            else                                                         \
+                L(LPB, false);                                           \
+            return hipGetLastError();                                    \
+        }                                                                \
     }
     FUSED_LPB(X)
 #undef X
+#undef L
     return hipErrorInvalidValue;
 }
 

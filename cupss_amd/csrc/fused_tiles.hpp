@@ -48,7 +48,7 @@ __host__ __device__ constexpr int tile_stride(int nc, int lpb)
     return rs;
 }
 
-template <int NC, int LPB, int MAXR = 3>
+template <int NC, int LPB, int MAXR = 3, bool SINGLE = false>
 struct FRowCfg {
     static constexpr int E = MAXR > 3 ? (NC >= 4 ? 4 : NC) : (NC >= 1024 ? 16 : (NC == 256 ? 8 : (NC >= 4 ? 4 : NC)));
     static constexpr int T = NC / E;
@@ -57,11 +57,13 @@ struct FRowCfg {
     // Two fields, and two products, at a time through their transforms: half
     // the barriers of a line over several wavefronts and one line's LDS
     // latency under the other's butterflies.  us per step, Gray-Scott 64^2
-    // 16.3 -> 15.9, 128^2 16.3 -> 15.1, 256^2 16.7 -> 16.0, 1024x512 26.3 ->
-    // 25.1.  Not the wide kernel, whose LDS and registers are the limit of a
-    // batch: model H 1024^2 alone 64.7 -> 63.8, but a mixed batch 122 -> 128.
-    // Not 16 elements a lane (registers).
-    static constexpr bool PAIR = MAXR > 1 && MAXR <= 3 && E <= 8;
+    // 16.7 -> 16.3, 128^2 15.9 -> 15.5, 256^2 16.7 -> 16.2, 512^2 24.2 -> 23.5,
+    // 1024x512 25.8 -> 25.2, and the same gain in batches of up to 256 of the
+    // short rows.  Launches of many long rows take them singly (SINGLE, with
+    // the same bits), see frows_n.  Not the wide kernel, whose LDS and
+    // registers are the limit of a batch: model H 1024^2 alone 64.7 -> 63.8,
+    // but a mixed batch 122 -> 128.  Not 16 elements a lane (registers).
+    static constexpr bool PAIR = !SINGLE && MAXR > 1 && MAXR <= 3 && E <= 8;
     static constexpr int LEN = (PAIR ? 2 : 1) * LPB * RS;
     static constexpr bool valid()
     {
@@ -248,12 +250,12 @@ __device__ __forceinline__ void r2c_pair(float2 (&v)[2][E], float2 *L, int ls, i
 // copy the twiddle tables into tws (2NC points) and tst (the NC-point
 // transform's stage tables) first (otherwise they are there already).
 // Ends with a workgroup barrier: the tile and the rows written are free.
-template <int NC, int LPB, int MAXR>
+template <int NC, int LPB, int MAXR, bool SINGLE = false>
 __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t step_rel,
                                            const float2 *__restrict__ sets, bool load_tw, float2 *tws, float2 *tst,
                                            float2 *tile)
 {
-    using C = FRowCfg<NC, LPB, MAXR>;
+    using C = FRowCfg<NC, LPB, MAXR, SINGLE>;
     constexpr int E = C::E, T = C::T, RS = C::RS, TH = C::THREADS;
     static_assert(T % 2 == 0 && E % 2 == 0, "noise lanes are paired");
     const int sy = a.g.sy;
