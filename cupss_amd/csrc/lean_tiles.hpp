@@ -22,21 +22,9 @@
 
 namespace cupss {
 
-// These tiles must give the same bits in every kernel that inlines them (a
-// run resumed by another kernel equals an uninterrupted one), but which
-// products the compiler fuses into additions depends on the code around
-// them.  Values pass opaquely in and out of each transform, and a*b + c is
-// fused within one expression only.
+// As the general tiles these must give the same bits in every kernel that
+// inlines them; here a*b + c is also fused within one expression only.
 #pragma clang fp contract(on)
-template <int E>
-__device__ __forceinline__ void opaque(float2 (&v)[E])
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-#pragma unroll
-    for (int e = 0; e < E; e++) asm("" : "+v"(v[e].x), "+v"(v[e].y));
-#endif
-}
-
 typedef uint32_t vu16 __attribute__((ext_vector_type(16)));
 
 // the lean program and phi's buffers of instance a, in scalar registers

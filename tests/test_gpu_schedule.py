@@ -1,6 +1,8 @@
-"""The tiles that a batch's size classes take without timing runs."""
+"""The tiles that a batch's size classes take without timing runs, and that no
+choice of tiles changes a bit."""
 import re
 
+import numpy as np
 import pytest
 
 import cupss_amd as C
@@ -52,3 +54,32 @@ def test_timed_kernel_is_the_one_launched(spec, name):
     s.profile_kernel(True)
     s.step(4)
     assert s.kernel_time()[2] == name
+
+
+def rect(spec, w, h):
+    rng = np.random.default_rng(12)
+    init = {f: rng.uniform(0.1, 0.5, w * h).astype(np.float32) for f, dyn in spec["fields"] if dyn}
+    return dict(spec, dims=(w, h, 1), init=init)
+
+
+def three_fields():
+    spec = spec_kpz(8)
+    return dict(spec, terms=spec["terms"] + [("h", ["h", "h"], [(-0.1,)]), ("h", ["h"], [(-0.05,)])])
+
+
+@pytest.mark.parametrize("kind", [lambda: spec_gray_scott(8), three_fields, lambda: spec_kpz(8)],
+                         ids=["two fields", "three fields", "lean"])
+@pytest.mark.parametrize("dims", [(512, 32), (1024, 32), (2048, 32), (4096, 32), (2048, 256), (32, 2048)])
+def test_tuned_and_default_tiles_give_equal_bits(kind, dims):
+    got = []
+    for autotune in (True, False, True):
+        b = C.Batch(autotune=autotune)
+        s, ids = build_system(C.System, C.pres, rect(kind(), *dims))
+        b.add(s)
+        b.step(9)
+        print(dims, autotune, b.schedule().split("\n")[0], flush=True)
+        got.append({f: s.get_real(i) for f, i in ids.items()})
+        b.close()
+        s.close()
+    for f in got[0]:
+        assert np.array_equal(got[0][f], got[1][f]) and np.array_equal(got[0][f], got[2][f]), f
