@@ -741,16 +741,17 @@ static int class_tables(const FusedBatch &B, const FusedBatch::Class &c, int lpb
 // 1024-point columns: 16 KPZ systems of 256^2 21.9 us a step against 19.9,
 // 4 of model H 1024^2 172 against 149)
 //
-// 128^2 with up to three real fields: 4 rows and 2 columns, not timed.  Of
-// every shape tried (2,2 .. 16,2) they are within 2 per cent of the best for 1
-// to 512 instances of Cahn-Hilliard, KPZ, Gray-Scott and a three-field system
-// (KPZ alone 12.8 us a step, 8 rows 13.3; 512 of them 72.8 and 72.9), and the
-// timing runs cost a new system half a millisecond, its first 16 steps' worth
-// over one workgroup an instance.
+// 128^2 with up to three real fields: 2 columns and 4 rows, 8 rows from 64
+// instances on, not timed.  Of every shape tried (2,2 .. 16,2) they are within
+// 2 per cent of the best for 1 to 512 instances of Cahn-Hilliard, KPZ,
+// Gray-Scott and a three-field system (us a step with 4 / 8 rows: KPZ alone
+// 12.8 / 13.3, 32 of them 15.4 / 15.3, 64 18.8 / 18.6, 128 28.1 / 27.7, 512
+// 72.8 / 72.9), and the timing runs cost a new system half a millisecond, its
+// first 16 steps' worth over one workgroup an instance.
 static void default_shapes(FusedBatch::Class &c)
 {
     if (c.nc == 64 && c.ny == 128 && c.width <= 3) {
-        c.lpb = 4;
+        c.lpb = c.insts.size() < 64 ? 4 : 8;
         c.twd = 2;
         c.fixed = true;
         return;
