@@ -434,13 +434,15 @@ static int make_ops(cupss_system s, FusedInst &a)
     return CUPSS_OK;
 }
 
-// an upper bound from the plan: every operator that is not a single monomial
-// without 1/|q|, and the updates with 1/|q|
+// an upper bound from the plan: every operator that lean_op refuses, and every
+// update that implicit_poly refuses
 size_t fused_table_bytes(cupss_system s)
 {
     const FusedPlan &P = s->plan;
     if (!P.ok || s->g.sz > 1) return 0;
-    auto plain = [](const std::vector<cupss_pres> &v) { return v.size() == 1 && v[0].invq == 0; };
+    auto plain = [](const std::vector<cupss_pres> &v) {
+        return v.size() == 1 && v[0].invq == 0 && v[0].iqz == 0 && v[0].q2n >= 0 && v[0].iqx >= 0 && v[0].iqy >= 0;
+    };
     size_t n = 0;
     for (auto &grp : P.groups) n += !plain(grp.pres);
     for (int d : P.derived) n += !plain(s->t[s->f[d].terms[0]].pres);
@@ -449,7 +451,7 @@ size_t fused_table_bytes(cupss_system s)
         for (int t : F.terms)
             if (s->t[t].fac.size() < 2) n += !plain(s->t[t].pres);
         bool poly = true;
-        for (auto &q : F.imp) poly = poly && q.invq == 0 && q.q2n <= 3;
+        for (auto &q : F.imp) poly = poly && q.invq == 0 && q.q2n >= 0 && q.q2n <= 3;
         n += !poly;
     }
     return sizeof(float) * (size_t)s->g.nh * n;
