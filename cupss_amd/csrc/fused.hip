@@ -562,11 +562,11 @@ hipError_t fused_cols_launch(int ny, int twd, int stored, const FusedInst *inst,
 // 64^2: one workgroup takes the steps in one launch, without a kernel boundary
 // per pass; on 128^2 one CU's vector issue is the bound and two launches per
 // step over the chip are faster.  us per step, one workgroup / two launches:
-// CH 64^2 5.9 / 8.2, KPZ 64^2 11.8 / 12.9, Gray-Scott 64^2 16.6 / 18.0; KPZ
-// 128^2 42 / 16, Gray-Scott 128^2 48 / 21 (two launches now take 12.5 and 15.1,
-// see FRowCfg and FColCfg).  Many instances at once hide either
-// (512 EW/KPZ instances: 169 us per step with 128^2 on one workgroup each or
-// not).
+// CH 64^2 5.9 / 8.2, KPZ 64^2 11.8 / 12.9, Gray-Scott 64^2 16.6 / 18.0; 128^2:
+// KPZ alone 43 / 12.5, 64 of them 43.6 / 18.6, 512 91 / 73; Gray-Scott alone
+// 49 / 15.4, 64 50 / 21.6.  Only where the instances just fill the CUs is one
+// workgroup each the better choice there: 256 of Gray-Scott 53 / 56, of
+// Cahn-Hilliard 25.7 / 26.6, of KPZ 48 / 45.
 bool fused_small_class(int nc, int ny, int width) { return width <= 3 && nc == 32 && ny == 64; }
 
 template <int NC, int N>

@@ -30,8 +30,14 @@ namespace cupss {
 // fields (the host checks).
 
 // Rows of 128 complex points take 8 elements a lane, not the 4 of the 2D tile
-// (FRowCfg): a large box fills the chip with rows, so the fewer exchanges win
-// (CH 256^3: 163.5 us per step with 4, 158.8 with 8).
+// (FRowCfg); shorter ones 4.  us per step with 4 / 8 elements (CH, and model B
+// with real-space noise after the comma): rows of 128 points, 256x32x32 22.4 /
+// 22.7, 26.8 / 29.0; 256x64x64 28.6 / 29.0, 38.2 / 39.5; 256x128x128 53.7 /
+// 52.0, 71.5 / 70.6; 256^3 162 / 156.5, 225 / 218: eight from 256x128x128 on,
+// which is where a step costs most.  Rows of 64 points, 128x32x32 21.5 / 22.3,
+// 25.0 / 27.7; 128^3 37.6 / 38.1, 48.3 / 50.6; 128x256x256 88.0 / 85.6, 120.2 /
+// 120.0: four.  (The elements set the order of a line's stages; one choice per
+// length keeps them apart from the other sides of the box.)
 template <int NC, int LPB, int MAXR>
 struct F3RowCfg {
     static constexpr int E = NC == 128 && MAXR <= 3 ? 8 : FRowCfg<NC, LPB, MAXR>::E;

@@ -22,8 +22,11 @@ namespace cupss {
 // stays inside one wavefront.  Many instances at once prefer fewer exchanges.
 // us per step with 8 -> 4 elements on rows of 64 and 128 complex points and
 // columns of 128 and 256 points: CH 256^2 10.2 -> 8.3, KPZ 128^2 16.3 -> 12.5,
-// Gray-Scott 256^2 20.2 -> 16.2, model H 256^2 39.7 -> 36.1; 512 EW/KPZ
-// instances of 64^2 .. 512^2 170 -> 174, CH 256^3 156 -> 161.  Rows of 256
+// Gray-Scott 256^2 20.2 -> 16.2, model H 256^2 39.7 -> 36.1, 16 of Gray-Scott
+// 256^2 26.6 -> 22.1; 64 of them 54 -> 57, 64 of a three-field system 256^2
+// 46.8 -> 50, 512 EW/KPZ instances of 64^2 .. 512^2 170 -> 174, CH 256^3
+// 156 -> 161.  The elements set the order of a line's stages, so they cannot
+// follow the number of instances: a system has the same bits in any batch.  Rows of 256
 // complex points stay at 8 (with 4: KPZ 512^2 20.3 -> 17.7, but the 512
 // instances 170 -> 183), and so do columns of 512 (with 4, two wavefronts
 // each: 18.3 and 188).  Longer lines take 4 over several wavefronts: 1024-point
