@@ -800,10 +800,15 @@ extern "C" int cupss_system_advance(cupss_system s, int nsteps)
     if (nsteps <= 0) return CUPSS_OK;
     // Real-space noise in 3D: a caller's graph records the general program's
     // launches, which need no set-up (the fused step's first run uploads its
-    // descriptor and allocates, and a recorded step has its counters fixed
-    // either way).
-    const bool general = s->plan.ok && s->g.sz > 1 && s->noise_mode == 0 && s->f[s->plan.phi].noisy &&
-                         recording(s->stream);
+    // descriptor, and a recorded step has its counters fixed either way).
+    // The graph may be replayed at any time and reads the dealiased copies,
+    // whose buffers fused runs use: such a system stays with the general
+    // program.
+    bool general = false;
+    if (s->plan.ok && s->g.sz > 1 && s->noise_mode == 0 && s->f[s->plan.phi].noisy) {
+        s->recorded = s->recorded || recording(s->stream);
+        general = s->recorded;
+    }
     if (s->path_mode == 0 && s->plan.ok && !general && !hooks_present(s) && fused_noise_ok(s)) {
         // a stale dealiased copy is consumed by one general step first
         if (fused_stale(s)) {

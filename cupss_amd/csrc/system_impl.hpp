@@ -120,6 +120,7 @@ struct cupss_system_t {
     // cupss_system_stat: steps by the fused path and by the 1D kernel, layouts
     // of the 1D program
     long fused_steps = 0, line_steps = 0, line_plans = 0;
+    bool recorded = false;    // a caller's graph holds general steps of it (3D, real-space noise)
     uint64_t step = 0;
     int device = 0;
     void *batch = nullptr;    // internal one-instance fused batch

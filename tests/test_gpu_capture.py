@@ -186,3 +186,30 @@ def test_recorded_line_goes_on():
         assert np.array_equal(s.get_real(i), twin.get_real(tid[f])), f
     s.close()
     st.close()
+
+
+def test_recorded_box_goes_on_between_direct_runs():
+    """Direct runs between replays leave what the recorded general steps read
+    as they expect it.  (The replayed steps draw the noise of the steps that
+    were recorded.)"""
+    spec = box((32, 32, 32))
+    st = Stream()
+    s, ids = build_system(C.System, C.pres, spec)
+    C.check(s.L.cupss_system_set_stream(s.h, st.s))
+    ex = st.record(lambda: s.step(2))
+    st.replay(ex)
+    s.step(2)
+    st.replay(ex)
+    s.step(1)
+    twin, tid = build_system(C.System, C.pres, spec)
+    twin.set_path(1)
+    twin.step(4)
+    C.check(twin.L.cupss_system_set_step(twin.h, 0))
+    twin.step(2)
+    C.check(twin.L.cupss_system_set_step(twin.h, 4))
+    twin.step(1)
+    for f, i in ids.items():
+        want = twin.get_real(tid[f])
+        assert np.linalg.norm(s.get_real(i) - want) <= 1e-5 * np.linalg.norm(want), f
+    s.close()
+    st.close()
