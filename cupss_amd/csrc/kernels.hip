@@ -341,10 +341,13 @@ static void launch_cols(int dir, bool mask, int p, const float2 *in, float2 *out
 }
 
 // widest valid tile that still gives >= 1024 workgroups, else the narrowest;
-// lines of 1024 points and more stay at 4 (32 adjacent bytes a row): 129
-// workgroups of 4 lines move a 1024^2 half spectrum faster than 513 of one
-// (general program, Cahn-Hilliard, us per step: 1024^2 52 -> 48, 2048^2
-// 112 -> 94), while 512^2 takes 32 with 2 lines and 33 with 4
+// lines of 1024 points and more stay at 4 (32 adjacent bytes a row) where that
+// leaves 100 workgroups: 129 of 4 lines move a 1024^2 half spectrum faster than
+// 513 of one, but on narrow grids the chip is idle.  General program,
+// Cahn-Hilliard, us per step with 1 or 2 / 4 lines: 1024^2 (129 workgroups of
+// 4) 52 / 48, 2048^2 112 / 93, 32x32x1024 (136) 68.8 / 63.7; 512x1024 (65)
+// 39.3 / 39.8, 256x2048 (33) 40.3 / 47.6, 64x2048 (9) 33.7 / 41.5, 16x16x2048
+// (36) 59.0 / 64.5; and 512^2 32 with 2 lines, 33 with 4
 template <int N>
 static void cols_n(int dir, bool mask, int p, const float2 *in, float2 *out, long ncols, long stride, long bstride,
                    long nbatch, const Geom &g, hipStream_t s, const float2 *tw)
@@ -354,7 +357,8 @@ static void cols_n(int dir, bool mask, int p, const float2 *in, float2 *out, lon
     for (int w : widths) {
         if (!ColCfg<N>::valid(w)) continue;
         pick = w;
-        if ((ncols + w - 1) / w * nbatch >= 1024 || (N >= 1024 && w == 4)) break;
+        const long groups = (ncols + w - 1) / w * nbatch;
+        if (groups >= 1024 || (N >= 1024 && w == 4 && groups >= 100)) break;
     }
     switch (pick) {
     case 64:
