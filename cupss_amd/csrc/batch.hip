@@ -103,6 +103,7 @@ struct FusedBatch {
     uint32_t once = 0;  // the last catch-up inside a caller's graph (FusedInst::caught)
     hipStream_t stream = nullptr;
     bool own_stream = false;
+    bool callers = false;  // the stream is a caller's, who may record it
 
     struct Class {
         int nc = 0, ny = 0;
@@ -847,13 +848,18 @@ static int build(FusedBatch &B)
     return CUPSS_OK;
 }
 
+// whether the batch's launches go into a caller's graph.  Asked of callers'
+// streams only: the runtime looks the stream up among all there are, 5 us with
+// 512 systems alive, which a one-step run of theirs would notice.
+static bool recording(const FusedBatch &B) { return B.callers && recording(B.stream); }
+
 // bring the device descriptors up to the steps taken: before anything but
 // step launches reads them, and before some of them are uploaded anew
 static int catch_up(FusedBatch &B)
 {
     if (B.lag == 0) return CUPSS_OK;
     const int ni = (int)B.h.size();
-    const uint32_t once = recording(B.stream) ? ++B.once : 0;
+    const uint32_t once = recording(B) ? ++B.once : 0;
     if (once != 0)
         for (FusedInst &a : B.h) a.caught = once;
     hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni, B.lag, once);
@@ -1358,7 +1364,7 @@ static int run(FusedBatch &B, int nsteps)
         mirror_run_end(B.h, (uint32_t)done);
     }
     if (nsteps > done) {
-        B.recorded = B.recorded || recording(B.stream);
+        B.recorded = B.recorded || recording(B);
         // offsets from the descriptors as the device holds them
         if (B.recorded || (uint64_t)B.lag + (uint64_t)(nsteps - done) > (1u << 30))
             if (int r = catch_up(B)) return r;
@@ -1513,6 +1519,7 @@ int fused_steps(cupss_system s, int nsteps)
         B->stream = s->stream;
         s->batch = B;
     }
+    B->callers = !s->own_stream;
     if (s->g.sz > 1) {
         B->stream = s->stream;
         return nsteps > 0 ? run3d(*B, s, nsteps) : CUPSS_OK;
@@ -1564,6 +1571,7 @@ extern "C" int cupss_batch_create(void *hip_stream, cupss_batch *out)
     cupss_batch b = new cupss_batch_t();
     if (hip_stream) {
         b->b.stream = (hipStream_t)hip_stream;
+        b->b.callers = true;
     } else {
         if (hipStreamCreateWithFlags(&b->b.stream, hipStreamNonBlocking) != hipSuccess) {
             delete b;

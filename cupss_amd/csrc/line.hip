@@ -553,7 +553,7 @@ bool line_eligible(cupss_system s)
     // the upload cannot be recorded into a graph: a caller's capture that
     // starts before the program was uploaded records the general program's
     // launches
-    return (S->gen == s->gen && S->vgen == s->vgen) || !recording(s->stream);
+    return (S->gen == s->gen && S->vgen == s->vgen) || s->own_stream || !recording(s->stream);
 }
 
 template <int NC, bool TAB>

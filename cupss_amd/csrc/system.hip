@@ -806,7 +806,7 @@ extern "C" int cupss_system_advance(cupss_system s, int nsteps)
     // program.
     bool general = false;
     if (s->plan.ok && s->g.sz > 1 && s->noise_mode == 0 && s->f[s->plan.phi].noisy) {
-        s->recorded = s->recorded || recording(s->stream);
+        s->recorded = s->recorded || (!s->own_stream && recording(s->stream));
         general = s->recorded;
     }
     if (s->path_mode == 0 && s->plan.ok && !general && !hooks_present(s) && fused_noise_ok(s)) {
