@@ -759,6 +759,11 @@ static void default_shapes(FusedBatch::Class &c)
         c.fixed = true;
         return;
     }
+    if (c.nc == 32 && c.ny == 64 && c.lean) {  // launch_class: runs of one step
+        c.lpb = 8;
+        c.twd = 8;
+        return;
+    }
     const std::vector<int> rs = fused_row_shapes(c.nc, c.ny, c.width), cs = fused_col_shapes(c.ny);
     c.lpb = rs.empty() ? 0 : rs.front();
     for (int v : rs)
@@ -957,7 +962,12 @@ static int launch_class(FusedBatch &B, size_t ci, int n0, int k, int rel0, hipSt
 {
     auto &c = B.classes[ci];
     const bool timed = B.profile && (int)ci == B.pclass && c.chunks.size() == 1;
-    if (c.small) {
+    // A run of one step of up to 128 simple 64^2 systems takes row and column
+    // launches: one workgroup each pays once it has its code and tables at
+    // hand, or has the chip full of others.  us a call of one step, one
+    // workgroup an instance / two launches: CH 12.1 / 8.1, KPZ 18.2 / 12.9, 16
+    // of KPZ 29.8 / 23.8, 256 35.9 / 34.5; of two steps, 256 of KPZ 48.8 / 52.
+    if (c.small && !(c.lean && k == 1 && c.insts.size() <= 128 && !B.profile)) {
         unsigned long long *ts = nullptr;
         if (timed && B.pcount < FusedBatch::PROF_SLOTS) {
             ts = B.pts + (size_t)(B.pcount++) * FUSED_TS_SLOTS * FUSED_TS_STRIDE;

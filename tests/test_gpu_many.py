@@ -49,3 +49,31 @@ def test_members_equal_the_system_alone(make, w, h, members):
     b.close()
     for s, _ in keep:
         s.close()
+
+
+@pytest.mark.parametrize("members", [3, 128, 129])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_one_step_runs_of_small_simple_systems(members, mode):
+    """64^2: runs of one step of up to 128 instances take two launches, longer
+    ones and those of more instances one workgroup each."""
+    print("one-step runs", members, mode, flush=True)
+    b = C.Batch()
+    keep = [build_system(C.System, C.pres, spec_kpz(64, seed=3 + i % 4)) for i in range(members)]
+    for s, _ in keep:
+        s.set_noise_mode(mode)
+        b.add(s)
+    runs = (1, 1, 4, 1, 2, 1)
+    for k in runs:
+        b.step(k)
+    for k in (0, 1, 2, members - 1):
+        for whole in ((sum(runs),), runs):
+            alone, aid = build_system(C.System, C.pres, spec_kpz(64, seed=3 + k % 4))
+            alone.set_noise_mode(mode)
+            for n in whole:
+                alone.step(n)
+            s, ids = keep[k]
+            for f, i in ids.items():
+                assert np.array_equal(s.get_real(i), alone.get_real(aid[f])), (k, f, whole)
+    b.close()
+    for s, _ in keep:
+        s.close()
