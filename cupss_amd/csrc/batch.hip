@@ -1011,6 +1011,14 @@ static int launch_all(FusedBatch &B, int n0, int k, int rel0)
         B.pcount = 0;
         HIP_TRY(fused_ts_reset_launch(B.pts, FusedBatch::PROF_SLOTS, B.stream));
     }
+    auto elementwise = [&](hipStream_t st) -> int {
+        if (B.neb > 0) HIP_TRY(fused_elem_launch(B.d, B.eb, B.neb, n0 & 1, (uint32_t)(n0 - rel0), k, st));
+        if (B.nleb > 0) HIP_TRY(lean_elem_launch(B.d, B.leb, B.nleb, n0 & 1, (uint32_t)(n0 - rel0), k, st));
+        return CUPSS_OK;
+    };
+    // one kind of work (a single system): no lanes to spread it over
+    if (B.classes.empty()) return elementwise(B.stream);
+    if (B.classes.size() == 1 && B.neb + B.nleb == 0) return launch_class(B, 0, n0, k, rel0, B.stream);
     std::vector<std::pair<double, int>> items;  // (cost, class index; -1 = elementwise)
     for (size_t ci = 0; ci < B.classes.size(); ci++) {
         double cost = 0;
@@ -1057,9 +1065,8 @@ static int launch_all(FusedBatch &B, int n0, int k, int rel0)
         hipStream_t st = lane[it] == 0 ? B.stream : B.lanes[lane[it] - 1];
         if (items[it].second >= 0) {
             if (int r = launch_class(B, (size_t)items[it].second, n0, k, rel0, st)) return r;
-        } else {
-            if (B.neb > 0) HIP_TRY(fused_elem_launch(B.d, B.eb, B.neb, n0 & 1, (uint32_t)(n0 - rel0), k, st));
-            if (B.nleb > 0) HIP_TRY(lean_elem_launch(B.d, B.leb, B.nleb, n0 & 1, (uint32_t)(n0 - rel0), k, st));
+        } else if (int r = elementwise(st)) {
+            return r;
         }
     }
     for (int j = 1; j < L; j++) {
