@@ -50,8 +50,8 @@ namespace cupss {
 // the parity and the counters (FusedBatch::lag).  One-step runs of 256^2
 // diffusion: 6.4 us with a launch per run, 4.0 without.
 //
-// once != 0: a launch inside a caller's graph that must take effect at the
-// graph's first replay only.
+// once != 0: one of several launches, in callers' graphs and direct, of which
+// the first to run takes effect.
 __global__ void k_bump_steps(FusedInst *inst, int n, uint32_t by, uint32_t once)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -100,7 +100,11 @@ struct FusedBatch {
     // any time: the offsets in those launches count from descriptors that
     // hold every step, so no run lets them lag any more.
     bool recorded = false;
-    uint32_t once = 0;  // the last catch-up inside a caller's graph (FusedInst::caught)
+    // The catch-up that the first such recording needed (FusedInst::caught):
+    // it stands at the head of every recording and of the first direct use
+    // after them, since nobody knows which of them runs first.
+    uint32_t once = 0, once_lag = 0;
+    bool once_open = false;
     hipStream_t stream = nullptr;
     bool own_stream = false;
     bool callers = false;  // the stream is a caller's, who may record it
@@ -777,7 +781,7 @@ static int build(FusedBatch &B)
 {
     B.release_tables();
     B.lag = 0;  // every descriptor is uploaded anew
-    B.recorded = false;  // a caller's graph of runs on the released tables cannot be replayed
+    B.recorded = B.once_open = false;  // a caller's graph of runs on the released tables cannot be replayed
     B.h.resize(B.sys.size());
     for (size_t i = 0; i < B.sys.size(); i++)
         if (int r = describe(B.sys[i], B.h[i])) return r;
@@ -858,19 +862,36 @@ static int build(FusedBatch &B)
 // 512 systems alive, which a one-step run of theirs would notice.
 static bool recording(const FusedBatch &B) { return B.callers && recording(B.stream); }
 
+static int bump(FusedBatch &B, uint32_t by, uint32_t once)
+{
+    const int ni = (int)B.h.size();
+    hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni, by, once);
+    HIP_TRY(hipGetLastError());
+    return CUPSS_OK;
+}
+
+// the catch-up of a recording that may not have been replayed yet
+static int take_once(FusedBatch &B)
+{
+    if (!B.once_open) return CUPSS_OK;
+    if (int r = bump(B, B.once_lag, B.once)) return r;
+    B.once_open = recording(B);
+    return CUPSS_OK;
+}
+
 // bring the device descriptors up to the steps taken: before anything but
 // step launches reads them, and before some of them are uploaded anew
 static int catch_up(FusedBatch &B)
 {
     if (B.lag == 0) return CUPSS_OK;
-    const int ni = (int)B.h.size();
-    const uint32_t once = recording(B) ? ++B.once : 0;
-    if (once != 0)
-        for (FusedInst &a : B.h) a.caught = once;
-    hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni, B.lag, once);
+    const uint32_t lag = B.lag;
     B.lag = 0;
-    HIP_TRY(hipGetLastError());
-    return CUPSS_OK;
+    if (!recording(B)) return bump(B, lag, 0);
+    B.once++;
+    B.once_lag = lag;
+    B.once_open = true;
+    for (FusedInst &a : B.h) a.caught = B.once;
+    return take_once(B);
 }
 
 static bool stale_tables(const FusedBatch &B)
@@ -1272,6 +1293,7 @@ static int settle(FusedBatch &B, int nsteps)
 static int flush(FusedBatch &B)
 {
     if (!B.settle_pending) return CUPSS_OK;
+    if (int r = take_once(B)) return r;
     B.settle_pending = false;
     // the final state is `lag` steps after the descriptors', the last step's
     // start in the other buffer
@@ -1299,6 +1321,7 @@ int fused_flush(cupss_system s)
 static int run(FusedBatch &B, int nsteps)
 {
     if (nsteps <= 0) return CUPSS_OK;
+    if (int r = take_once(B)) return r;
     // a member whose state another batch's run left column-major: written
     // back first
     for (cupss_system s : B.sys)
@@ -1352,11 +1375,7 @@ static int run(FusedBatch &B, int nsteps)
         if (!B.gexec) {
             HIP_TRY(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
             int rc = launch_all(B, 0, K, 0);
-            if (rc == CUPSS_OK) {
-                const int ni = (int)B.h.size();
-                hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni,
-                                   (uint32_t)K, 0u);
-            }
+            if (rc == CUPSS_OK) rc = bump(B, (uint32_t)K, 0);
             hipGraph_t g = nullptr;
             HIP_TRY(hipStreamEndCapture(B.stream, &g));
             if (rc != CUPSS_OK) {
@@ -1391,9 +1410,7 @@ static int run(FusedBatch &B, int nsteps)
         // buffer order: they follow the steps
         B.lag += (uint32_t)(nsteps - done);
         if (B.recorded) {
-            const int ni = (int)B.h.size();
-            hipLaunchKernelGGL(k_bump_steps, dim3((ni + 255) / 256), dim3(256), 0, B.stream, B.d, ni, B.lag, 0u);
-            HIP_TRY(hipGetLastError());
+            if (int r = bump(B, B.lag, 0)) return r;
             B.lag = 0;
         }
         mirror_run_end(B.h, (uint32_t)(nsteps - done));

@@ -99,6 +99,35 @@ def test_replayed_runs_go_on(name, before, n):
     st.close()
 
 
+@pytest.mark.parametrize("before", [1, 2, 5])
+@pytest.mark.parametrize("name", list(SYSTEMS))
+def test_recordings_in_any_order(name, before):
+    """Two recordings one after the other, a direct run before either is
+    replayed, the second replayed first."""
+    print("capture order", name, before, flush=True)
+    st = Stream()
+    s, ids = make(name)
+    C.check(s.L.cupss_system_set_stream(s.h, st.s))
+    s.step(1)
+    s.step(before)
+    two = st.record(lambda: s.step(2))
+    four = st.record(lambda: s.step(4))
+    if before != 2:
+        s.step(1)
+    st.replay(four)
+    st.replay(two)
+    s.step(1)
+    st.replay(two)
+    s.step(2)
+    got = {f: s.get_real(i) for f, i in ids.items()}
+    twin, tid = make(name)
+    twin.step(1 + before + (before != 2) + 4 + 2 + 1 + 2 + 2)
+    for f in got:
+        assert np.array_equal(got[f], twin.get_real(tid[f])), f
+    s.close()
+    st.close()
+
+
 def test_replayed_runs_of_a_batch_go_on():
     """Members with transforms, of one workgroup each and elementwise; two
     recorded runs of different lengths."""
