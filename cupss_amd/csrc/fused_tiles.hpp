@@ -194,7 +194,8 @@ __device__ __forceinline__ void c2r_prep(const float2 (&xa)[E], const float2 (&y
 // The tiles must give the same bits in every kernel that inlines them (any
 // tile shape, one workgroup or many, a run resumed by another kernel), but
 // which products the compiler fuses into which additions depends on the code
-// around them: values pass opaquely in and out of each transform.
+// around them: values pass opaquely in and out of a transform where that was
+// seen to differ (rows of 16 elements a lane; the lean tiles).
 template <int E>
 __device__ __forceinline__ void opaque(float2 (&v)[E])
 {
@@ -328,9 +329,7 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
             // the row's part of the tile becomes its transform's LDS (the
             // row's lanes are the only ones that read or write it from here)
             line_sync<(T <= 64)>();
-#pragma unroll
-            for (int m = 0; m < P; m++)
-                if (m == 0 || two) opaque(v[m]);
+            if constexpr (E > 8) opaque(v[0]);
             if constexpr (P == 2) {
                 if (two)
                     fft_pair<NC, E, +1, false, (T <= 64)>(v, L, TS, t, tst);
@@ -342,7 +341,7 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
 #pragma unroll
             for (int m = 0; m < P; m++)
                 if (f + m < MAXR && (m == 0 || two)) {
-                    opaque(v[m]);
+                    if constexpr (E > 8) opaque(v[m]);
 #pragma unroll
                     for (int e = 0; e < E; e++) r[f + m < MAXR ? f + m : 0][e] = cscale(v[m][e], a.scale);
                 }
@@ -385,8 +384,6 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
             float2 v[2][E];
             products(gi, v[0]);
             products(gi + 1, v[1]);
-            opaque(v[0]);
-            opaque(v[1]);
             r2c_pair<NC, E, T>(v, L, TS, t, tws, tst);
             tile_store<NC, LPB, RS, TH>(a.X[gi], tile, sy, y0);
             tile_store<NC, LPB, RS, TH>(a.X[gi + 1], tile + TS, sy, y0);
@@ -395,7 +392,7 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
     for (; gi < a.ngroups; gi++) {
         float2 v[E];
         products(gi, v);
-        opaque(v);
+        if constexpr (E > 8) opaque(v);
         r2c_tile<NC, E, T, TW_STAGE>(v, L, t, tws, tst);
         tile_store<NC, LPB, RS, TH>(a.X[gi], tile, sy, y0);
         __syncthreads();
@@ -439,7 +436,7 @@ __device__ __forceinline__ void frows_tile(const FusedInst &a, int y0, uint32_t 
             v[e2] = even ? own : rcv;
             v[e2 + E / 2] = even ? rcv : own;
         }
-        opaque(v);
+        if constexpr (E > 8) opaque(v);
         r2c_tile<NC, E, T, TW_STAGE>(v, L, t, tws, tst);
         tile_store<NC, LPB, RS, TH>(eta, tile, sy, y0);
         __syncthreads();  // the tile is the next source's transform LDS
