@@ -1362,7 +1362,7 @@ static int run(FusedBatch &B, int nsteps)
         for (cupss_system s : B.sys)
             if (s->stream != B.stream) HIP_TRY(hipStreamSynchronize(s->stream));
     if (int r = refresh(B)) return r;
-    if (!twiddle_sets(B.stream)) return fail(CUPSS_ERR_NOMEM, "twiddle tables");
+    if (!B.classes.empty() && !twiddle_sets(B.stream)) return fail(CUPSS_ERR_NOMEM, "twiddle tables");
     if (int r = launch_prologue(B)) return r;
     if (B.autotune && !B.tuned && !B.classes.empty()) {
         B.drop_graph();
@@ -1525,7 +1525,8 @@ static int run3d(FusedBatch &B, cupss_system s, int nsteps)
         unsigned long long *ts = nullptr;
         if (B.profile && B.pcount < FusedBatch::PROF_SLOTS)
             ts = B.pts + (size_t)(B.pcount++) * FUSED_TS_SLOTS * FUSED_TS_STRIDE;
-        HIP_TRY(fused3d_z_launch(g.sz, B.twd3, B.d, g.nc1, g.sy, par0 ^ (i & 1), rel0 + (uint32_t)i, 1, i > 0, st, ts));
+        HIP_TRY(fused3d_z_launch(g.sz, B.twd3, B.d, g.nc1, g.sy, par0 ^ (i & 1), rel0 + (uint32_t)i,
+                                 a.nreal > 0 ? 1 : 2, i > 0, st, ts));
         HIP_TRY(inverse_y());
     }
     // the kx = 0, sx/2 planes of the final state (partners are in other z

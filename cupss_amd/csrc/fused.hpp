@@ -269,9 +269,9 @@ struct F3yArgs {
     int n, nc1, sz;
 };
 hipError_t fused3d_y_launch(const Geom &g, int dir, F3yArgs a, hipStream_t s);
-// mode 0: prologue (W_f of the current state), 1: step; herm: phi's kx = 0
-// and sx/2 planes are not yet Hermitian, project them on reading; ts as for
-// fused_cols_launch
+// mode 0: prologue (W_f of the current state), 1: step, 2: step of a system
+// without real fields; herm: phi's kx = 0 and sx/2 planes are not yet
+// Hermitian, project them on reading; ts as for fused_cols_launch
 hipError_t fused3d_z_launch(int nz, int twd, const FusedInst *inst, int nc1, int sy, int parity, uint32_t step_rel,
                             int mode, int herm, hipStream_t s, unsigned long long *ts = nullptr);
 // derived fields from phi's spectrum [parity], natural layout

@@ -420,31 +420,33 @@ __global__ __launch_bounds__((F3zCfg<N, TWD>::THREADS)) __attribute__((amdgpu_wa
 #pragma unroll
         for (int e = 0; e < E; e++) nw[e] = cur[e];
     }
-    // W_f = IFFT_z(mask_f * L_f * phi) on the lines the mask keeps
-    const int ny = ky > g.sy / 2 ? ky - g.sy : ky;
-    for (int f = 0; f < a.nreal; f++) {
-        if (kx0 > a.kmax[f] || abs(ny) > a.kymax[f]) continue;  // uniform over the workgroup
-        const int lz = a.p[f] > 0 ? g.sz / (a.p[f] + 1) : g.sz;
-        const bool zero = !upd && a.zero[f] != 0;
-        float2 v[E];
-        const TermRefDev &LM = a.lmul[f];
-        float lm[E];
-        if (LM.npres > 0) multiplier_line<E>(a.pool, LM.pres0, LM.npres, LM.mult_i, lb, lm);
+    if (mode != 2) {
+        // W_f = IFFT_z(mask_f * L_f * phi) on the lines the mask keeps
+        const int ny = ky > g.sy / 2 ? ky - g.sy : ky;
+        for (int f = 0; f < a.nreal; f++) {
+            if (kx0 > a.kmax[f] || abs(ny) > a.kymax[f]) continue;  // uniform over the workgroup
+            const int lz = a.p[f] > 0 ? g.sz / (a.p[f] + 1) : g.sz;
+            const bool zero = !upd && a.zero[f] != 0;
+            float2 v[E];
+            const TermRefDev &LM = a.lmul[f];
+            float lm[E];
+            if (LM.npres > 0) multiplier_line<E>(a.pool, LM.pres0, LM.npres, LM.mult_i, lb, lm);
 #pragma unroll
-        for (int e = 0; e < E; e++) {
-            const int kz = t + e * T;
-            const int nz = kz > g.sz / 2 ? kz - g.sz : kz;
-            const bool keep = !zero && kx <= a.kmax[f] && abs(nz) <= lz;
-            const float2 w = LM.npres > 0 ? apply_mult(lm[e], LM.mult_i, nw[e]) : nw[e];
-            v[e] = keep ? w : make_float2(0.f, 0.f);
-        }
-        fft_line<N, E, +1, TW_STAGE, false, (TWD * T <= 64)>(v, L, t, tws);
-        if (active && kx <= a.kmax[f]) {
-            float2 *__restrict__ w = a.W[f];
+            for (int e = 0; e < E; e++) {
+                const int kz = t + e * T;
+                const int nz = kz > g.sz / 2 ? kz - g.sz : kz;
+                const bool keep = !zero && kx <= a.kmax[f] && abs(nz) <= lz;
+                const float2 w = LM.npres > 0 ? apply_mult(lm[e], LM.mult_i, nw[e]) : nw[e];
+                v[e] = keep ? w : make_float2(0.f, 0.f);
+            }
+            fft_line<N, E, +1, TW_STAGE, false, (TWD * T <= 64)>(v, L, t, tws);
+            if (active && kx <= a.kmax[f]) {
+                float2 *__restrict__ w = a.W[f];
 #pragma unroll
-            for (int e = 0; e < E; e++) gstore(w, base + (long)(t + e * T) * plane, v[e]);
+                for (int e = 0; e < E; e++) gstore(w, base + (long)(t + e * T) * plane, v[e]);
+            }
+            line_sync<(TWD * T <= 64)>();
         }
-        line_sync<(TWD * T <= 64)>();
     }
     if (slot) {
         __syncthreads();
